@@ -70,7 +70,8 @@ struct LayerState {
 // below were measured best on the 64.3M-edge power-law graph
 // (100 -> 8x32 -> 8x32 -> 1x47, max in-degree 17 000): the sum form keeps
 // many short chunks, the one-row-per-wave 8-head kernel fewer, longer ones,
-// and the one-head kernel (8 rows per wave) splits only its heaviest rows.
+// and the row-group kernel (64 edges a step on its heavy rows) splits only its
+// heaviest rows.
 // Small graphs (below kSmallGraphEdges edges) split more rows into shorter
 // chunks, 512/256 for every kernel: their heaviest rows are a larger share of
 // a short launch (169K-node, 2.5M-edge power-law graph: 0.88 ms against 1.23
@@ -79,9 +80,9 @@ struct LayerState {
 // kMaxChunksPerRow chunks: each chunk reduces the maxima of all chunks of its
 // row and the last one adds all partial sums, so many chunks per row cost
 // more than they balance.  The 8-head kernel (one row per wave) scales min
-// with the chunk; the sum form (32-row tiles) and the one-head kernel (8 rows
-// per wave) hold a heavy row's neighbours at the same pace, and split from
-// twice the chunk instead.  On the 100M-edge R-MAT graph (max in-degree
+// with the chunk; the sum form (32-row tiles) holds a heavy row's neighbours
+// at the same pace, and it and the row-group kernel split from twice the chunk
+// instead.  On the 100M-edge R-MAT graph (max in-degree
 // 132 270) that gives 6144/2048 (8-head) and 4096/2048 (sum form, one head),
 // the best of measured sweeps there (sum form: 7.4 ms against 8.4 at
 // 8192/2048).
@@ -155,7 +156,7 @@ struct gatgpu_ctx {
     gatgpu::DevBuf xorig;  // the features in original node order (x32 is their sorted-order copy)
     gatgpu::LayerState L[3];
     // options (in-degree thresholds)
-    uint32_t block_min = 512;        // rows >= this take a block
+    uint32_t block_min = 512;        // rows below this are never split
     uint32_t split_min = 0;          // user option: rows >= this are split (0: per-kernel defaults)
     uint32_t split_chunk = 0;        // user option: edges per chunk (0: per-kernel defaults)
     bool keep_xbf = false;           // option GATGPU_OPT_KEEP_INPUT_BF16

@@ -67,9 +67,10 @@ int bind(gatgpu_ctx* c) {
 
 // Sorted-position boundaries of the degree bins.
 int compute_bins(gatgpu_ctx* c) {
-    // Thresholds: block bin, each plan's split degree, then the short rows.
-    uint32_t thr[2 + kPlans] = {c->block_min ? c->block_min - 1 : 0};
+    // Thresholds: block bin, each plan's split degree, the short rows, the wave rows.
+    uint32_t thr[3 + kPlans] = {c->block_min ? c->block_min - 1 : 0};
     thr[1 + kPlans] = kShortDeg;
+    thr[2 + kPlans] = (c->e < kWaveDegEdges ? kWaveDegSmall : kWaveDeg) - 1;
     uint32_t maxdeg = 0;  // degrees are sorted ascending
     if (c->n) HIPCHECK(c, hipMemcpy(&maxdeg, c->sorted_deg + (c->n - 1), 4, hipMemcpyDeviceToHost));
     const bool small = c->e < kSmallGraphEdges;
@@ -83,20 +84,20 @@ int compute_bins(gatgpu_ctx* c) {
         P.chunk = c->split_chunk ? c->split_chunk : chunk0 * f;
         thr[1 + q] = P.min - 1;
     }
-    // block_min 0 means every row takes a block.
     HIPCHECK(c, c->small.ensure(128));
-    // small[]: [0,4) max degree, [8,16) neighbor steps, [16,36) thresholds, [40,80) positions
+    // small[]: [0,4) max degree, [8,16) neighbor steps, [16,40) thresholds, [40,88) positions
     uint32_t* dthr = reinterpret_cast<uint32_t*>(c->small.as<char>() + 16);
     uint64_t* dpos = reinterpret_cast<uint64_t*>(c->small.as<char>() + 40);
     HIPCHECK(c, hipMemcpyAsync(dthr, thr, sizeof(thr), hipMemcpyHostToDevice, c->stream));
-    HIPCHECK(c, launch_count_le(c->sorted_deg, c->n, dthr, 2 + kPlans, dpos, c->stream));
-    uint64_t pos[2 + kPlans];
+    HIPCHECK(c, launch_count_le(c->sorted_deg, c->n, dthr, 3 + kPlans, dpos, c->stream));
+    uint64_t pos[3 + kPlans];
     HIPCHECK(c, hipMemcpyAsync(pos, dpos, sizeof(pos), hipMemcpyDeviceToHost, c->stream));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     RowBins b;
     b.n = c->n;
     b.block_begin = c->block_min ? pos[0] : 0;
     b.short_end = pos[1 + kPlans];
+    b.wave_begin = pos[2 + kPlans];
     c->bins = b;
     std::vector<uint64_t> prow;
     for (int q = 0; q < kPlans; ++q) {
@@ -677,15 +678,15 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
     a.e = c->e;
     a.r_from_z = pa.r_from_z;
     a.ar = Ls.ar.as<float>();
-    const bool one_head = !fixed && !aggregate_vec_supported(a) && aggregate_k1_supported(a);
-    if (one_head && a.out32) {
+    const bool grouped = !fixed && !aggregate_vec_supported(a);
+    if (grouped && K == 1 && a.out32) {
         a.out_perm = b.out_perm;
         a.ostride = b.ostride;
     }
     if (done) done->out_perm_used = a.out_perm != nullptr;
-    // The one-head kernel takes its own split plan; the 8-head, generic and
-    // fixed-p kernels the 8-head one.
-    const SplitPlan& P = c->plans[one_head ? kPlanOne : kPlanVec];
+    // The row-group kernel takes its own split plan; the 8-head and fixed-p
+    // kernels the 8-head one.
+    const SplitPlan& P = c->plans[grouped ? kPlanOne : kPlanVec];
     SplitTable t = P.table;
     if (b.mchunk) t.mchunk = b.mchunk;
     if (b.part) t.part = b.part;

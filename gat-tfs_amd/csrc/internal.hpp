@@ -241,11 +241,21 @@ void pack_projection_f32(const float* w, const float* blr, int in, int heads, in
 // Rows of at most this many edges share the sum form's 16-edge batches (four
 // rows a batch).
 constexpr uint32_t kShortDeg = 4;
+// aggregate.hip: rows of at least this many edges take a wave each.  A wave
+// takes 64 edges a step (8 groups of 8 lanes), so shorter rows leave its loads
+// idle, and longer ones left to a group are a chain of batches that outlasts
+// the launch.  Forward with the line at 16 / 32 / 64 / 128 edges: 64.3M edges
+// 20.94 / 19.63 / 19.41 / 19.39 ms, 2.5M edges 1164 / 1151 / 1149 / 1154 us,
+// 20K rows of 8 edges (at most 170) 122 / 122 / 132 / 153 us, where the launch
+// does not fill the chip and only the chain counts.
+constexpr uint32_t kWaveDeg = 64, kWaveDegSmall = 32;
+constexpr uint64_t kWaveDegEdges = 1u << 21;  // graphs of fewer edges take kWaveDegSmall
 struct RowBins {
-    // Sorted positions [0, n) split by degree: [0, block_begin) one wave per
-    // row, [block_begin, split_begin) one block per row, [split_begin, n)
-    // several blocks per row.  [0, short_end): rows of at most kShortDeg edges.
-    uint64_t block_begin = 0, split_begin = 0, n = 0, short_end = 0;
+    // Sorted positions split by degree: [0, short_end): rows of at most
+    // kShortDeg edges; [wave_begin, n): of kWaveDeg edges or more;
+    // [split_begin, n): cut into chunks (never below block_begin, the first
+    // row of GATGPU_OPT_BLOCK_ROW_MIN_DEGREE edges).
+    uint64_t block_begin = 0, split_begin = 0, n = 0, short_end = 0, wave_begin = 0;
 };
 struct AggArgs {
     const uint64_t* prow;
@@ -301,14 +311,10 @@ hipError_t launch_split_prescan(const uint64_t* prow, const uint32_t* pcol, cons
 // edge order, [e][K]) and fixture denominators ([n][K]); writes den and out32.
 hipError_t launch_aggregate_fixed(const AggArgs& a, const float* p_sorted, const float* den_fixture,
                                   const RowBins& bins, const SplitTable& split, hipStream_t s);
-// aggregate_k1.hip: one head, rows of at most 64 features.
-bool aggregate_k1_supported(const AggArgs& a);
-// Row stride (floats) of the one-head kernel's FP32 rows written to original
-// node order: the kernel's widest row (G lanes x 16 bytes, 128 or 256 bytes),
-// padded with zeros past the W classes.
+// Row stride (floats) of a one-head layer's FP32 rows written to original
+// node order: the group's widest row (128 or 256 bytes), padded with zeros past
+// the W classes.
 int k1_out_stride(bool feat_bf16, int W);
-hipError_t launch_aggregate_k1(const AggArgs& a, const RowBins& bins, const SplitTable& split,
-                               hipStream_t s);
 // aggregate_af.hip: aggregate-first bf16 layer (input rows <= 128, 32 features per head).
 struct AfArgs {
     const uint64_t* prow;

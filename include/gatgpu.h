@@ -115,7 +115,8 @@ typedef struct gatgpu_times {
 
 /* Options (gatgpu_set_option).  Thresholds are in-degrees. */
 enum {
-    GATGPU_OPT_BLOCK_ROW_MIN_DEGREE = 1, /* rows at/above use a block per row  */
+    GATGPU_OPT_BLOCK_ROW_MIN_DEGREE = 1, /* rows below are never split (default
+                                            512; 0: no such limit)           */
     GATGPU_OPT_SPLIT_ROW_MIN_DEGREE = 2, /* rows at/above are split over waves
                                             (default per kernel: 1024 sum form,
                                             1536 8-head, 2048 one-head; 512 on
@@ -130,7 +131,7 @@ enum {
                                             16M edges; scaled as above; a value
                                             >= 64 applies to all, 0 restores) */
     /* 4 is not a key: rows of small degree take one wave each like the rest
-       (the one-head kernel already packs 8 rows of equal degree per wave). */
+       (or share one with rows of equal degree, where a row needs fewer lanes). */
     GATGPU_OPT_KEEP_INPUT_BF16 = 5,      /* 1: bf16 transform-first layers also
                                             store the input rows their
                                             projection rounds (stage XBF);
