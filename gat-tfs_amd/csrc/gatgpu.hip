@@ -633,23 +633,25 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
             pa.x = srcbf;
         }
         HIPCHECK(c, launch_projection_mfma(pa, c->stream, c->cus));
-    } else if (projection_f32_supported(D, K, dim)) {
-        // FP32 MFMA: Z = X W and L/R = X B_LR (FP32 products and sums)
+    } else if (Ls.wpk32.p) {
         ProjF32Args fa{};
         fa.x = src32;
         fa.n = n;
         fa.in = D;
         fa.xs = D;
-        fa.wpk = Ls.wpk32.as<float>();
-        fa.head_blocks = (W + 31) / 32;
+        fa.wpk = Ls.wpk32.as<uint4>();
+        fa.w32 = Ls.w32.as<float>();
+        fa.al = Ls.al.as<float>();
+        fa.ar = Ls.ar.as<float>();
         fa.width = W;
         fa.heads = K;
+        fa.dim = dim;
         fa.z = static_cast<float*>(b.z);
         fa.zs = zs;
         fa.left = b.left;
         fa.right = b.right;
         fa.tiles = (n + 31) / 32;
-        HIPCHECK(c, launch_projection_f32(fa, c->stream));
+        HIPCHECK(c, launch_projection_split(fa, c->stream, c->cus));
     } else {
         HIPCHECK(c, launch_projection(src32, nullptr, Ls.w32.as<float>(), n, D, K, dim, Ls.al.as<float>(),
                                       Ls.ar.as<float>(), static_cast<float*>(b.z), nullptr, b.left, b.right,
@@ -870,20 +872,9 @@ int gatgpu_set_layer(gatgpu_ctx* c, int layer, int in, int heads, int dim, const
     L.heads = heads;
     L.dim = dim;
     // Static preparation (prepare(), baseline/src/common.cpp:97-119): bf16
-    // copy of W (kept as FP32 values) and B_LR = W a for the reordered front end.
-    std::vector<float> wq(wn), blr(size_t(in) * 2 * heads);
+    // copy of W (kept as FP32 values); B_LR = W a goes into the packed blocks.
+    std::vector<float> wq(wn);
     for (uint64_t i = 0; i < wn; ++i) wq[i] = bf16_widen(bf16_rne(w[i]));
-    for (int k = 0; k < in; ++k)
-        for (int h = 0; h < heads; ++h) {
-            float l = 0, r = 0;
-            for (int d = 0; d < dim; ++d) {
-                const float wv = w[size_t(k) * W + h * dim + d];
-                l += wv * al[h * dim + d];
-                r += wv * ar[h * dim + d];
-            }
-            blr[size_t(k) * 2 * heads + h] = l;
-            blr[size_t(k) * 2 * heads + heads + h] = r;
-        }
     std::vector<uint16_t> packed;
     pack_projection_weights(wq.data(), al, ar, in, heads, dim, packed, L.ksteps, L.groups, L.nmb);
     HIPCHECK(c, L.wpk.ensure(packed.size() * 2));
@@ -897,17 +888,15 @@ int gatgpu_set_layer(gatgpu_ctx* c, int layer, int in, int heads, int dim, const
     HIPCHECK(c, L.wq32.ensure(wn * 4));
     HIPCHECK(c, L.al.ensure(W * 4));
     HIPCHECK(c, L.ar.ensure(W * 4));
-    HIPCHECK(c, L.blr.ensure(blr.size() * 4));
     HIPCHECK(c, hipMemcpyAsync(L.w32.p, w, wn * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(c, hipMemcpyAsync(L.wq32.p, wq.data(), wn * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(c, hipMemcpyAsync(L.al.p, al, W * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(c, hipMemcpyAsync(L.ar.p, ar, W * 4, hipMemcpyHostToDevice, c->stream));
-    HIPCHECK(c, hipMemcpyAsync(L.blr.p, blr.data(), blr.size() * 4, hipMemcpyHostToDevice, c->stream));
-    std::vector<float> f32pk;
-    if (projection_f32_supported(in, heads, dim)) {
-        pack_projection_f32(w, blr.data(), in, heads, dim, f32pk);
-        HIPCHECK(c, L.wpk32.ensure(f32pk.size() * 4));
-        HIPCHECK(c, hipMemcpyAsync(L.wpk32.p, f32pk.data(), f32pk.size() * 4, hipMemcpyHostToDevice, c->stream));
+    if (const size_t split_bytes = projection_split_bytes(w, in, heads, dim)) {
+        HIPCHECK(c, L.wpk32.ensure(split_bytes));
+        HIPCHECK(c, launch_pack_split(L.w32.as<float>(), in, heads, dim, L.wpk32.p, c->stream));
+    } else {
+        L.wpk32.release();
     }
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     L.set = true;

@@ -174,10 +174,9 @@ hipError_t launch_projection(const float* x32, const uint16_t* xbf, const float*
                              int in, int heads, int dim, const float* al, const float* ar,
                              float* z32, uint16_t* zbf, float* left, float* right, float* zscratch,
                              int zs, hipStream_t s);
-// L/R only (aggregate-first front end): LR = X B_LR with B_LR = W a.
-hipError_t launch_lr_reordered(const float* x32, const uint16_t* xbf, const float* blr,
-                               uint64_t n, int in, int heads, float* left, float* right,
-                               hipStream_t s);
+// L and R as dots of the FP32 Z rows (lr_from_z).
+hipError_t launch_lr_from_z(const float* z, uint64_t n, int heads, int dim, int zs, const float* al, const float* ar,
+                            float* left, float* right, hipStream_t s);
 
 // projection_mfma.hip: bf16 MFMA projection with the fused L/R block.
 struct ProjArgs {
@@ -220,22 +219,30 @@ hipError_t launch_projection_mfma(const ProjArgs& a, hipStream_t s, int cus);
 void pack_lr_weights(const float* wq, const float* al, const float* ar, int in, int heads, int dim,
                      std::vector<uint16_t>& out, int& ksteps);
 
-// FP32 projection on the MFMA units (projection_mfma.hip).
+// projection_split.hip: the FP32 projection on the bf16 MFMA units, each operand
+// split into three bf16 parts.
 struct ProjF32Args {
-    const float* x;      // [n][xs] FP32 input, xs == in
+    const float* x;      // [n][xs] FP32 input, any alignment and width; nothing past a row's `in` values is read
     uint64_t n;
     int in, xs;
-    const float* wpk;    // pack_projection_f32() order
-    int head_blocks, width, heads;
+    const uint4* wpk;    // launch_pack_split() order
+    const float* w32;    // [in][width]: the products of rows the split cannot carry
+    const float* al;     // aL, aR [width]
+    const float* ar;
+    int width, heads, dim;
     float* z;            // [n][zs] FP32 output
     int zs;
     float* left;         // [n][heads]
     float* right;        // [n][heads]
     uint64_t tiles;      // ceil(n / 32)
+    // set by the launch: the k range and output blocks of one kernel launch
+    int k0, kn, nob;
+    bool add;
 };
-bool projection_f32_supported(int in, int heads, int dim);
-hipError_t launch_projection_f32(const ProjF32Args& a, hipStream_t s);
-void pack_projection_f32(const float* w, const float* blr, int in, int heads, int dim, std::vector<float>& out);
+hipError_t launch_projection_split(ProjF32Args a, hipStream_t s, int cus);
+size_t projection_split_bytes(const float* w, int in, int heads, int dim);
+// w: device [in][heads * dim]; out: projection_split_bytes.
+hipError_t launch_pack_split(const float* w, int in, int heads, int dim, void* out, hipStream_t s);
 
 // aggregate.hip
 // Rows of at most this many edges share the sum form's 16-edge batches (four

@@ -3,10 +3,8 @@
 //
 // Reference: projection (baseline/src/baseline_standard.cpp:3-6, one all-head
 // GEMM, cblas_sgemm or cblas_gemm_bf16bf16f32), lr_from_z (:7-20) and the
-// FP32 -> bf16 RNE convert (baseline/src/common.cpp:80-93).  The reordered
-// front end LR = X (W a) of the aggregate-first path follows lr_reordered
-// (baseline_standard.cpp:29-43) and prepare_attention
-// (implementation/src/gat_tfs_online.cpp:48-73).
+// FP32 -> bf16 RNE convert (baseline/src/common.cpp:80-93).  Takes the FP32
+// layers whose weights projection_split.hip cannot carry.
 #include "internal.hpp"
 
 namespace gatgpu {
@@ -95,37 +93,40 @@ k_gemm_tiled(const float* __restrict__ x32, const uint16_t* __restrict__ xbf, co
     }
 }
 
-// One thread per (row, head): the dots of lr_from_z, then the optional bf16 store of Z.
+// G lanes per (row, head): the dots of lr_from_z over the FP32 Z row, VEC
+// features a load.  Bound by the reads of Z, so consecutive lanes read
+// consecutive features: one lane per dot, reading its head's features one by
+// one, took 142 us on 120K rows of 8 x 32 (0.9 TB/s).
+template <int VEC, int G>
 __global__ void __launch_bounds__(kThreads)
 k_lr_from_z(const float* __restrict__ z, uint64_t n, int K, int dim, int zs, const float* __restrict__ al,
             const float* __restrict__ ar, float* __restrict__ left, float* __restrict__ right) {
-    const uint64_t t = blockIdx.x * uint64_t(kThreads) + threadIdx.x;
-    if (t >= n * K) return;
+    const uint64_t q = blockIdx.x * uint64_t(kThreads) + threadIdx.x, t = q / G;
+    const int sub = int(q % G);
+    if (t >= n * K) return;  // whole groups
     const uint64_t i = t / K;
     const int h = int(t % K);
     const float* zi = z + i * zs + h * dim;
     float l = 0.0f, r = 0.0f;
-    for (int d = 0; d < dim; ++d) {
-        l += zi[d] * al[h * dim + d];
-        r += zi[d] * ar[h * dim + d];
+    for (int f = sub * VEC; f < dim; f += G * VEC) {
+        float v[VEC];
+        __builtin_memcpy(v, __builtin_assume_aligned(zi + f, 4 * VEC), 4 * VEC);
+#pragma unroll
+        for (int x = 0; x < VEC; ++x)
+            if (f + x < dim) {  // (a one-head row's last vector reaches into its padding)
+                l += v[x] * al[h * dim + f + x];
+                r += v[x] * ar[h * dim + f + x];
+            }
     }
-    left[t] = l;
-    right[t] = r;
-}
-
-// One thread per (row, column of B_LR): LR = X B_LR, B_LR = [b_L | b_R] [D][2K].
-__global__ void __launch_bounds__(kThreads)
-k_lr_reordered(const float* __restrict__ x32, const uint16_t* __restrict__ xbf,
-               const float* __restrict__ blr, uint64_t n, int D, int K, float* __restrict__ left,
-               float* __restrict__ right) {
-    const uint64_t t = blockIdx.x * uint64_t(kThreads) + threadIdx.x;
-    if (t >= n * 2 * K) return;
-    const uint64_t i = t / (2 * K);
-    const int c = int(t % (2 * K));
-    float s = 0.0f;
-    for (int k = 0; k < D; ++k) s += ldx(x32, xbf, i * D + k) * blr[size_t(k) * 2 * K + c];
-    if (c < K) left[i * K + c] = s;
-    else right[i * K + c - K] = s;
+#pragma unroll
+    for (int off = 1; off < G; off <<= 1) {
+        l += __shfl_xor(l, off);
+        r += __shfl_xor(r, off);
+    }
+    if (sub == 0) {
+        left[t] = l;
+        right[t] = r;
+    }
 }
 
 uint32_t grid_for(uint64_t items, uint32_t cap) {
@@ -152,6 +153,28 @@ hipError_t launch_widen_bf16(const uint16_t* x, float* y, uint64_t count, hipStr
     return hipGetLastError();
 }
 
+namespace {
+template <int VEC, int G>
+hipError_t lr_from_z_lanes(const float* z, uint64_t n, int heads, int dim, int zs, const float* al, const float* ar,
+                           float* left, float* right, hipStream_t s) {
+    const uint64_t blocks = (n * uint64_t(heads) * G + kThreads - 1) / kThreads;
+    if (blocks < 1 || blocks > 0x7fffffffu) return hipErrorInvalidValue;
+    k_lr_from_z<VEC, G><<<dim3(uint32_t(blocks)), kThreads, 0, s>>>(z, n, heads, dim, zs, al, ar, left, right);
+    return hipGetLastError();
+}
+}  // namespace
+
+// 16-byte loads where every head starts on 16 bytes (rows do: zs % 4 == 0).
+hipError_t launch_lr_from_z(const float* z, uint64_t n, int heads, int dim, int zs, const float* al, const float* ar,
+                            float* left, float* right, hipStream_t s) {
+    const bool vec = zs % 4 == 0 && (dim % 4 == 0 || heads == 1);
+    if (vec)
+        return dim <= 8 ? lr_from_z_lanes<4, 2>(z, n, heads, dim, zs, al, ar, left, right, s)
+                        : lr_from_z_lanes<4, 8>(z, n, heads, dim, zs, al, ar, left, right, s);
+    return dim <= 8 ? lr_from_z_lanes<1, 2>(z, n, heads, dim, zs, al, ar, left, right, s)
+                    : lr_from_z_lanes<1, 8>(z, n, heads, dim, zs, al, ar, left, right, s);
+}
+
 hipError_t launch_projection(const float* x32, const uint16_t* xbf, const float* w, uint64_t n,
                              int in, int heads, int dim, const float* al, const float* ar,
                              float* z32, uint16_t* zbf, float* left, float* right, float* zscratch,
@@ -163,21 +186,9 @@ hipError_t launch_projection(const float* x32, const uint16_t* xbf, const float*
     k_gemm_tiled<<<grid, kThreads, 0, s>>>(x32, xbf, w, zf, n, in, W, zs);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    const uint64_t pairs = n * uint64_t(heads);
-    k_lr_from_z<<<dim3(uint32_t((pairs + kThreads - 1) / kThreads)), kThreads, 0, s>>>(zf, n, heads, dim, zs,
-                                                                                       al, ar, left, right);
-    if ((err = hipGetLastError()) != hipSuccess) return err;
+    if ((err = launch_lr_from_z(zf, n, heads, dim, zs, al, ar, left, right, s)) != hipSuccess) return err;
     if (zbf) return launch_to_bf16(zf, zbf, n * uint64_t(zs), s);
     return hipSuccess;
-}
-
-hipError_t launch_lr_reordered(const float* x32, const uint16_t* xbf, const float* blr,
-                               uint64_t n, int in, int heads, float* left, float* right,
-                               hipStream_t s) {
-    const uint64_t items = n * 2 * uint64_t(heads);
-    k_lr_reordered<<<dim3(uint32_t((items + kThreads - 1) / kThreads)), kThreads, 0, s>>>(
-        x32, xbf, blr, n, in, heads, left, right);
-    return hipGetLastError();
 }
 
 }  // namespace gatgpu
