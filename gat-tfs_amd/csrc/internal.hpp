@@ -159,6 +159,9 @@ hipError_t launch_relabel(const uint32_t* perm, const uint32_t* pcol, uint32_t* 
 // an index >= n_src gives a zero row).
 hipError_t launch_gather_rows(const void* src, uint64_t src_stride_words, void* dst, uint64_t dst_stride_words,
                               const uint32_t* idx, uint64_t rows, uint64_t n_src, uint32_t words, hipStream_t s);
+// Rows of `width` floats at stride `stride` to dense rows; dst (16-byte aligned)
+// may be host memory mapped to the device.
+hipError_t launch_pack_rows(const float* src, uint64_t stride, float* dst, uint64_t rows, uint32_t width, hipStream_t s);
 hipError_t launch_count_le(const uint32_t* sorted_deg, uint64_t n, const uint32_t* thresholds,
                            int count, uint64_t* positions, hipStream_t s);
 

@@ -269,6 +269,38 @@ k_gather_rows(const uint32_t* __restrict__ src, uint64_t src_stride, uint32_t* _
     }
 }
 
+// 16-byte stores in order (the reads are whole rows from the L2).  To mapped
+// host memory 53 to 55 GB/s, the copy engine's 56 less 10 us.
+constexpr uint32_t kPackRows = 64;
+__global__ void __launch_bounds__(kThreads)
+k_pack_rows(const float* __restrict__ src, uint64_t stride, float* __restrict__ dst, uint64_t rows, uint32_t width) {
+    const uint64_t chunks = (rows + kPackRows - 1) / kPackRows;
+    for (uint64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+        const uint64_t r0 = c * kPackRows;
+        const uint32_t total = uint32_t(rows - r0 < kPackRows ? rows - r0 : kPackRows) * width;
+        const float* s0 = src + r0 * stride;
+        float* d0 = dst + r0 * width;  // 64 rows: 16-byte aligned for any width
+        for (uint32_t t = 4 * threadIdx.x; t < total; t += 4 * kThreads) {
+            uint32_t r = t / width, w = t - r * width;
+            float v[4];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                v[x] = t + x < total ? s0[r * stride + w] : 0.0f;
+                if (++w == width) {
+                    w = 0;
+                    ++r;
+                }
+            }
+            if (t + 4 <= total) {
+                *reinterpret_cast<float4*>(d0 + t) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+                for (int x = 0; x < 3; ++x)
+                    if (t + x < total) d0[t + x] = v[x];
+            }
+        }
+    }
+}
+
 // neighbor_steps = sum over 16-row tiles of the last (= largest) degree.
 __global__ void __launch_bounds__(kThreads)
 k_neighbor_steps(const uint32_t* __restrict__ sorted_deg, uint64_t n, uint64_t* __restrict__ steps) {
@@ -384,6 +416,14 @@ hipError_t launch_gather_rows(const void* src, uint64_t src_stride_words, void* 
 hipError_t launch_neighbor_steps(const uint32_t* sorted_deg, uint64_t n, uint64_t* steps,
                                  hipStream_t s) {
     k_neighbor_steps<<<grid_for((n + 15) / 16, kThreads, 1024), kThreads, 0, s>>>(sorted_deg, n, steps);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_rows(const float* src, uint64_t stride, float* dst, uint64_t rows, uint32_t width,
+                            hipStream_t s) {
+    if (!rows) return hipSuccess;
+    k_pack_rows<<<grid_for((rows + kPackRows - 1) / kPackRows, 1, 2048), kThreads, 0, s>>>(src, stride, dst, rows,
+                                                                                         width);
     return hipGetLastError();
 }
 
