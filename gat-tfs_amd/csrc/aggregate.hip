@@ -82,7 +82,7 @@ struct GrpArgs {
     const float* R;
     const ZT* Z;
     int K, dim, W, zs;
-    bool hidden;
+    bool hidden, round_bf16;
     float* mx;
     float* den;
     float* out32;
@@ -300,6 +300,7 @@ __device__ inline void finish(const GrpArgs<typename C::ZT>& a, const Lane<C>& s
         for (int x = 0; x < V; ++x) {
             y[x] = s.acc[v][x] * scale;
             if (a.hidden) y[x] = elu(y[x]);
+            if (a.round_bf16) y[x] = bf16_widen(bf16_hw(y[x]));
         }
         const int f = s.off[v];
         if (a.out32 && a.os != a.W) {
@@ -449,6 +450,7 @@ hipError_t run(const AggArgs& g, const RowBins& bins, const SplitTable& t, hipSt
     a.W = W;
     a.zs = g.fstride;
     a.hidden = g.hidden;
+    a.round_bf16 = g.round_bf16;
     a.mx = g.mx;
     a.den = g.den;
     a.out32 = g.out32;

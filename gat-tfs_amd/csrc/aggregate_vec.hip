@@ -74,7 +74,7 @@ struct VArgs {
     const float* L;
     const float* R;
     const ZT* Z;
-    bool hidden;
+    bool hidden, round_bf16;
     float* mx;
     float* den;
     float* out32;
@@ -347,7 +347,7 @@ __device__ inline void aggregate(uint64_t beg, uint64_t end, const uint32_t* __r
 template <class C>
 __device__ inline void finish_row(uint32_t i, const float (&acc)[C::ACC], const float (&den)[C::VPL],
                                   const float (&M)[C::VPL], const int (&h)[C::VPL], int slot, int sub,
-                                  bool hidden, float* mx, float* dn, float* out32,
+                                  bool hidden, bool round_bf16, float* mx, float* dn, float* out32,
                                   uint16_t* outbf) {
     if (slot != 0) return;
 #pragma unroll
@@ -361,10 +361,10 @@ __device__ inline void finish_row(uint32_t i, const float (&acc)[C::ACC], const 
         float o[C::VEC];
 #pragma unroll
         for (int x = 0; x < C::VEC; ++x) o[x] = acc[v * C::VEC + x] * scale;
-        if (hidden && out32) {
+        if (hidden && out32 && !round_bf16) {
 #pragma unroll
             for (int x = 0; x < C::VEC; ++x) o[x] = elu(o[x]);
-        } else if (hidden) {  // stored as bf16 only
+        } else if (hidden) {  // stored as bf16, or as the values of bf16
 #pragma unroll
             for (int x = 0; x < C::VEC; ++x) o[x] = elu_bf16(o[x]);
         }
@@ -378,6 +378,10 @@ __device__ inline void finish_row(uint32_t i, const float (&acc)[C::ACC], const 
             else *reinterpret_cast<uint2*>(outbf + off) = make_uint2(w[0], w[1]);
         }
         if (out32) {
+            if (round_bf16) {
+#pragma unroll
+                for (int x = 0; x < C::VEC; ++x) o[x] = bf16_widen(bf16_hw(o[x]));
+            }
 #pragma unroll
             for (int x = 0; x < C::VEC; x += 4)
                 *reinterpret_cast<float4*>(out32 + off + x) = make_float4(o[x], o[x + 1], o[x + 2], o[x + 3]);
@@ -526,7 +530,7 @@ __device__ inline void run_chunk(const VArgs<ZT>& a, uint64_t c, int lane, int s
         }
     }
     if (lane == 0) a.sp.counter[first] = 0;  // ready for the next launch
-    finish_row<C>(i, tot, dtot, M, st.h, slot, sub, a.hidden, a.mx, a.den, a.out32, a.outbf);
+    finish_row<C>(i, tot, dtot, M, st.h, slot, sub, a.hidden, a.round_bf16, a.mx, a.den, a.out32, a.outbf);
 }
 
 // short_rows: the positions [0, short_rows) are k_agg_vec_short's.
@@ -562,7 +566,7 @@ __global__ void __launch_bounds__(kThreads) k_agg_vec(VArgs<ZT> a, uint64_t shor
     if (end == beg)
 #pragma unroll
         for (int v = 0; v < C::VPL; ++v) st.m[v] = 0.0f;
-    finish_row<C>(i, st.acc, st.den, st.m, st.h, slot, sub, a.hidden, a.mx, a.den, a.out32, a.outbf);
+    finish_row<C>(i, st.acc, st.den, st.m, st.h, slot, sub, a.hidden, a.round_bf16, a.mx, a.den, a.out32, a.outbf);
 }
 
 // Rows of at most kShortDeg edges, the sorted positions [0, a.short_rows), for
@@ -641,7 +645,7 @@ __global__ void __launch_bounds__(kThreads) k_agg_vec_short(VArgs<uint16_t> a, u
         merge_slots<C>(st[r]);
         if (cnt[r] == 0) st[r].m[0] = 0.0f;  // empty row: max 0, denominator 0, output 0
         if (ri[r] != kNone)
-            finish_row<C>(ri[r], st[r].acc, st[r].den, st[r].m, st[r].h, slot, sub, a.hidden, a.mx, a.den, a.out32,
+            finish_row<C>(ri[r], st[r].acc, st[r].den, st[r].m, st[r].h, slot, sub, a.hidden, a.round_bf16, a.mx, a.den, a.out32,
                           a.outbf);
     }
 }
@@ -836,7 +840,7 @@ bool offsets32(uint64_t n) {
 // their own.
 template <class C, class ZT>
 hipError_t run(const AggArgs& g, const RowBins& bins, const SplitTable& t, hipStream_t s) {
-    VArgs<ZT> a{g.prow, g.pcol, g.perm, g.left, g.right, static_cast<const ZT*>(g.feat), g.hidden, g.mx, g.den,
+    VArgs<ZT> a{g.prow, g.pcol, g.perm, g.left, g.right, static_cast<const ZT*>(g.feat), g.hidden, g.round_bf16, g.mx, g.den,
                 g.out32, g.outbf, g.n, g.e, bins.split_begin,
                 SplitArgs{t.chunks, t.chunk_k, t.chunk_first, t.chunk_edges, t.mchunk, t.part, t.counter}, g.ar};
     // (With R from Z the rows of 8 x 64 layers still take the short launch,
@@ -910,7 +914,7 @@ hipError_t launch_aggregate_vec_next(const AggArgs& g, const RowBins& bins, cons
                                      hipStream_t s) {
     if (!aggregate_vec_next_supported(g, f)) return hipErrorInvalidValue;
     using C = Cfg<uint16_t, 256, 8, kURz>;
-    VArgs<uint16_t> a{g.prow, g.pcol, g.perm, g.left, g.right, static_cast<const uint16_t*>(g.feat), g.hidden,
+    VArgs<uint16_t> a{g.prow, g.pcol, g.perm, g.left, g.right, static_cast<const uint16_t*>(g.feat), g.hidden, g.round_bf16,
                       g.mx, g.den, g.out32, g.outbf, g.n, g.e, bins.split_begin,
                       SplitArgs{t.chunks, t.chunk_k, t.chunk_first, t.chunk_edges, t.mchunk, t.part, t.counter},
                       g.ar};

@@ -119,6 +119,8 @@ struct TfBufs {
     uint32_t* counter = nullptr;
     bool fused_convert_ok = false;   // the FP32 input carries kF32Pad floats past its last row
     bool keep_xbf = false;           // write the rounded input rows to xbf even when the convert is fused
+    bool no_xbf = false;             // nobody reads the rounded input rows
+    bool round_bf16 = false;         // out32 gets the widened values of bf16-stored rows
     const uint32_t* out_perm = nullptr;  // one-head kernel: output row of sorted position k
     int ostride = 0;                     // its out32 row stride (floats)
     // The next layer's projection in this layer's aggregation epilogue
@@ -181,7 +183,7 @@ int hip_fail(gatgpu_ctx* c, const char* what, hipError_t e);
 // Row stride (elements) of Z for a layer of `heads` x `width / heads`.
 int z_stride(int precision, int heads, int width, bool* r_in_z);
 // What run_tf did: the FP32 input rows were rounded inside the projection
-// (then b.xbf holds them only with b.keep_xbf); the one-head kernel wrote
+// and not kept in b.xbf; the one-head kernel wrote
 // its rows through b.out_perm.
 struct TfDone {
     bool fused_convert = false;

@@ -585,7 +585,7 @@ int run_layer(gatgpu_ctx* c, int l, int precision, int dataflow, bool hidden, co
     Ls.outbf_valid = want_outbf && fuse != kFuseNext;
     Ls.out_original = done.out_perm_used;
     Ls.out_stride = done.out_perm_used ? ostride : W;
-    Ls.xbf_valid = bf16 && src32 && (!done.fused_convert || c->keep_xbf);
+    Ls.xbf_valid = bf16 && src32 && !done.fused_convert;
     Ls.xbf_stride = xs;
     return GATGPU_OK;
 }
@@ -630,9 +630,14 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
     // ---- convert (bf16 path, FP32 source only; a bf16 source was rounded in
     // the previous layer's epilogue, which equals convert() of that output).
     // Where the fast projection applies, the rounding happens in its loads.
-    const bool fused = !b.projected && bf16 && src32 && b.fused_convert_ok && D % 4 == 0 &&
-                       projection_fp32_input(pa);  // 16-byte aligned rows
-    if (done) done->fused_convert = fused;
+    const bool tile = !b.projected && bf16 && projection_tile_path(pa, src32 != nullptr, c->cus);
+    const bool in_loads = !b.projected && bf16 && src32 && b.fused_convert_ok && D % 4 == 0 &&
+                          projection_fp32_input(pa);  // 16-byte aligned rows
+    const bool fused = in_loads || (tile && src32);
+    // The rounded rows of a layer that has a convert of its own elsewhere are
+    // kept (stage XBF).
+    const bool keep_xbf = b.keep_xbf || (!in_loads && !b.no_xbf);
+    if (done) done->fused_convert = fused && !keep_xbf;
     if (b.projected) {
         // Z, L and R come from the previous layer's epilogue: no convert, no projection.
     } else if (bf16 && src32 && !fused) {
@@ -649,7 +654,7 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
             pa.x32 = src32;
             pa.xs = D;
             pa.in = D;
-            if (b.keep_xbf) {  // the rounded rows also leave the kernel
+            if (keep_xbf) {  // the rounded rows also leave the kernel
                 pa.xout = b.xbf;
                 pa.xouts = xs;
             }
@@ -703,6 +708,7 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
     a.n = c->n;
     a.e = c->e;
     a.r_from_z = pa.r_from_z;
+    a.round_bf16 = b.round_bf16;
     a.ar = Ls.ar.as<float>();
     const bool grouped = !fixed && !aggregate_vec_supported(a);
     if (grouped && K == 1 && a.out32) {

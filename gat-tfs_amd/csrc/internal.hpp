@@ -166,9 +166,8 @@ hipError_t launch_count_le(const uint32_t* sorted_deg, uint64_t n, const uint32_
                            int count, uint64_t* positions, hipStream_t s);
 
 // projection.hip
-hipError_t launch_to_bf16(const float* x, uint16_t* y, uint64_t count, hipStream_t s);
 hipError_t launch_widen_bf16(const uint16_t* x, float* y, uint64_t count, hipStream_t s);
-// x [n][d] FP32 -> y [n][dp] bf16 with zero columns d..dp-1.
+// x [n][d] FP32 -> y [n][dp] bf16 with zero columns d..dp-1 (dp a multiple of 4).
 hipError_t launch_to_bf16_pad(const float* x, uint16_t* y, uint64_t n, int d, int dp, hipStream_t s);
 // Z = X W with the L/R attention dots and the store of Z (FP32 or bf16).
 // X is FP32 (x32 != null) or bf16 bits (xbf != null); W is FP32 values (for
@@ -219,6 +218,12 @@ bool projection_fp32_input(const ProjArgs& a);
 void pack_projection_weights(const float* wq, const float* al, const float* ar, int in, int heads, int dim,
                              std::vector<uint16_t>& out, int& ksteps, int& groups, int& nmb);
 hipError_t launch_projection_mfma(const ProjArgs& a, hipStream_t s, int cus);
+// projection_tile.hip: one output block a wave; FP32 input of any width (x32 rows
+// of `in` values) or bf16.
+bool projection_tile_shape(const ProjArgs& a);
+hipError_t launch_projection_tile(const ProjArgs& a, hipStream_t s, int cus);
+// True when launch_projection_mfma takes that path.
+bool projection_tile_path(const ProjArgs& a, bool fp32_rows, int cus);
 void pack_lr_weights(const float* wq, const float* al, const float* ar, int in, int heads, int dim,
                      std::vector<uint16_t>& out, int& ksteps);
 
@@ -292,6 +297,9 @@ struct AggArgs {
     // Row stride of out32 (floats) where out_perm is set: k1_out_stride, so
     // that every scattered row is whole 128-byte lines.  0: W.
     int ostride = 0;
+    // out32 holds the values of bf16-stored rows (widened): the ELU of those and
+    // their rounding.
+    bool round_bf16 = false;
 };
 // The permuted column array carries kPcolPad zero entries past its e
 // edges, so that kernels may load a whole batch of wave-uniform source ids

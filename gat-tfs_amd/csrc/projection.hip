@@ -12,22 +12,28 @@ namespace {
 
 constexpr int kThreads = 256;
 
+// x [n][d] FP32 -> y [n][dp] bf16, columns d..dp-1 zero.  Bound by memory: four
+// columns a thread, 16 bytes in and 8 out (one column a thread: 271 us for 300K
+// rows of 500, 3.3 TB/s).
 __global__ void __launch_bounds__(kThreads)
-k_to_bf16(const float* __restrict__ x, uint16_t* __restrict__ y, uint64_t count) {
-    for (uint64_t i = blockIdx.x * uint64_t(kThreads) + threadIdx.x; i < count;
-         i += uint64_t(gridDim.x) * kThreads)
-        y[i] = bf16_rne(x[i]);
-}
-
-// x [n][d] FP32 -> y [n][dp] bf16, columns d..dp-1 zero.
-__global__ void __launch_bounds__(kThreads)
-k_to_bf16_pad(const float* __restrict__ x, uint16_t* __restrict__ y, uint64_t n, int d, int dp) {
-    const uint64_t count = n * uint64_t(dp);
+k_to_bf16_pad(const float* __restrict__ x, uint16_t* __restrict__ y, uint64_t n, uint32_t d, uint32_t dp) {
+    const uint32_t per_row = dp / 4;
+    const uint64_t count = n * uint64_t(per_row);
     for (uint64_t i = blockIdx.x * uint64_t(kThreads) + threadIdx.x; i < count;
          i += uint64_t(gridDim.x) * kThreads) {
-        const uint64_t r = i / dp;
-        const int c = int(i - r * dp);
-        y[i] = c < d ? bf16_rne(x[r * d + c]) : uint16_t(0);
+        const uint64_t r = i / per_row;
+        const uint32_t c = uint32_t(i - r * per_row) * 4;
+        const float* p = x + r * d + c;
+        float v[4] = {};
+        if (c + 4 <= d) {
+            __builtin_memcpy(v, p, 16);  // rows of any width: 4-byte alignment
+        } else {
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                if (c + q < d) v[q] = p[q];
+        }
+        *reinterpret_cast<uint2*>(y + r * dp + c) =
+            make_uint2(bf16_rne(v[0]) | uint32_t(bf16_rne(v[1])) << 16, bf16_rne(v[2]) | uint32_t(bf16_rne(v[3])) << 16);
     }
 }
 
@@ -137,14 +143,9 @@ uint32_t grid_for(uint64_t items, uint32_t cap) {
 
 }  // namespace
 
-hipError_t launch_to_bf16(const float* x, uint16_t* y, uint64_t count, hipStream_t s) {
-    k_to_bf16<<<grid_for(count, 1u << 16), kThreads, 0, s>>>(x, y, count);
-    return hipGetLastError();
-}
-
 hipError_t launch_to_bf16_pad(const float* x, uint16_t* y, uint64_t n, int d, int dp, hipStream_t s) {
-    if (dp == d) return launch_to_bf16(x, y, n * uint64_t(d), s);
-    k_to_bf16_pad<<<grid_for(n * uint64_t(dp), 1u << 16), kThreads, 0, s>>>(x, y, n, d, dp);
+    if (dp % 4 || dp < d) return hipErrorInvalidValue;
+    k_to_bf16_pad<<<grid_for(n * uint64_t(dp / 4), 1u << 16), kThreads, 0, s>>>(x, y, n, uint32_t(d), uint32_t(dp));
     return hipGetLastError();
 }
 
@@ -187,7 +188,7 @@ hipError_t launch_projection(const float* x32, const uint16_t* xbf, const float*
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     if ((err = launch_lr_from_z(zf, n, heads, dim, zs, al, ar, left, right, s)) != hipSuccess) return err;
-    if (zbf) return launch_to_bf16(zf, zbf, n * uint64_t(zs), s);
+    if (zbf) return launch_to_bf16_pad(zf, zbf, n, zs, zs, s);
     return hipSuccess;
 }
 

@@ -1134,7 +1134,20 @@ bool projection_fp32_input(const ProjArgs& a) {
            (wide_supported_impl(a) && a.ksteps == 8);
 }
 
+// Below 8 tiles per CU the fast path's blocks of 8 tiles leave CUs idle.  With
+// more tiles the shapes without a path of their own (3 to 7 output blocks, 9 to 15
+// and more than 16 k steps of one group) come here from FP32 rows, which
+// k_proj_mfma needs converted first (300K rows of 200 -> 4 x 32: 117 us against
+// 119 + 70); from bf16 rows it is the faster one (128 -> 4 x 32: 51 us against 59,
+// 1M rows of 512 -> 16: 322 against 392).
+bool projection_tile_path(const ProjArgs& a, bool fp32_rows, int cus) {
+    if (!projection_tile_shape(a)) return false;
+    return a.tiles < uint64_t(kWaves) * uint64_t(cus) ||
+           (fp32_rows && !fast_supported_impl(a) && !wide_supported_impl(a));
+}
+
 hipError_t launch_projection_mfma(const ProjArgs& a, hipStream_t s, int cus) {
+    if (projection_tile_path(a, a.x32 != nullptr, cus)) return launch_projection_tile(a, s, cus);
     if (a.x32 && !projection_fp32_input(a)) return hipErrorInvalidValue;
     if (a.r_from_z && a.heads == 1) return rz_one_head(a) && a.ar ? launch_wide(a, s, cus) : hipErrorInvalidValue;
     if (fast_supported_impl(a)) {
