@@ -381,26 +381,24 @@ __global__ void __launch_bounds__(kThreads) k_agg_rows(GrpArgs<typename C::ZT> a
                 for (int v = 0; v < C::VPL; ++v) {
                     if (s.off[v] >= a.W) continue;
 #pragma unroll
-                    for (int x = 0; x < C::VEC; ++x) part[s.off[v] + x] = s.acc[v][x];
+                    for (int x = 0; x + 1 < C::VEC; x += 2)
+                        store_coherent2(part + s.off[v] + x, s.acc[v][x], s.acc[v][x + 1]);
+                    if constexpr (C::VEC == 1) store_coherent(part + s.off[v], s.acc[v][0]);
                     if (s.lead[v]) {
-                        part[512 + s.head[v]] = s.d[v];
-                        part[520 + s.head[v]] = s.m[v];
+                        store_coherent(part + 512 + s.head[v], s.d[v]);
+                        store_coherent(part + 520 + s.head[v], s.m[v]);
                     }
                 }
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            uint32_t old = 0;
-            if (lane == 0)
-                old = __hip_atomic_fetch_add(a.counter + first, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            old = __shfl(old, 0);
-            if (old + 1 != nch) return;
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            if (arrive(a.counter + first, lane) + 1 != nch) return;
             // The row's maximum, then the groups take every GPW-th chunk each.
             const float* base = a.part + uint64_t(first) * kPartStride;
 #pragma unroll
             for (int v = 0; v < C::VPL; ++v) {
                 float M = -INFINITY;
-                for (uint32_t q = 0; q < nch; ++q) M = fmaxf(M, base[uint64_t(q) * kPartStride + 520 + s.head[v]]);
+#pragma unroll 16
+                for (uint32_t q = 0; q < nch; ++q)
+                    M = fmaxf(M, load_coherent(base + uint64_t(q) * kPartStride + 520 + s.head[v]));
                 s.m[v] = M;
                 s.d[v] = 0.0f;
 #pragma unroll
@@ -409,11 +407,16 @@ __global__ void __launch_bounds__(kThreads) k_agg_rows(GrpArgs<typename C::ZT> a
 #pragma unroll 4
                 for (uint32_t q = uint32_t(g); q < nch; q += C::GPW) {
                     const float* p = base + uint64_t(q) * kPartStride;
-                    const float mq = p[520 + s.head[v]];
+                    const float mq = load_coherent(p + 520 + s.head[v]);
                     const float sc = mq == M ? 1.0f : exp_w(mq - M);
-                    s.d[v] += p[512 + s.head[v]] * sc;
+                    s.d[v] += load_coherent(p + 512 + s.head[v]) * sc;
 #pragma unroll
-                    for (int x = 0; x < C::VEC; ++x) s.acc[v][x] += p[f + x] * sc;
+                    for (int x = 0; x + 1 < C::VEC; x += 2) {
+                        const float2 t = load_coherent2(p + f + x);
+                        s.acc[v][x] += t.x * sc;
+                        s.acc[v][x + 1] += t.y * sc;
+                    }
+                    if constexpr (C::VEC == 1) s.acc[v][0] += load_coherent(p + f) * sc;
                 }
             }
             merge_groups(s);

@@ -387,13 +387,13 @@ __device__ void afs_merge_row(const AfsArgs& a, uint64_t c, int l, float* sw) {
         float mx = -INFINITY;
 #pragma unroll 16
         for (uint32_t q = 0; q < nch; ++q) {
-            mref = fmaxf(mref, a.part[(c + q) * kPart + kMOff + l]);
-            mx = fmaxf(mx, a.part[(c + q) * kPart + kMxOff + l]);
+            mref = fmaxf(mref, load_coherent(a.part + (c + q) * kPart + kMOff + l));
+            mx = fmaxf(mx, load_coherent(a.part + (c + q) * kPart + kMxOff + l));
         }
 #pragma unroll 16
         for (uint32_t q = 0; q < nch; ++q) {
             const float* pq = a.part + (c + q) * kPart;
-            d += pq[kDenOff + l] * exp_w(pq[kMOff + l] - mref);
+            d += load_coherent(pq + kDenOff + l) * exp_w(load_coherent(pq + kMOff + l) - mref);
         }
         a.mx[uint64_t(i) * 8 + l] = mx;
         a.den[uint64_t(i) * 8 + l] = d * exp_w(mref - mx);  // against the exact max
@@ -423,8 +423,8 @@ __device__ void afs_merge_row(const AfsArgs& a, uint64_t c, int l, float* sw) {
 #pragma unroll
                 for (int h = 0; h < 8; ++h) {
                     const float* pq = a.part + (c + q0 + u) * kPart;
-                    v[u][h] = *reinterpret_cast<const float2*>(pq + 2 * l + h * 128);
-                    mq[u][h] = pq[kMOff + h];
+                    v[u][h] = load_coherent2(pq + 2 * l + h * 128);
+                    mq[u][h] = load_coherent(pq + kMOff + h);
                 }
 #pragma unroll
             for (uint32_t u = 0; u < CNT; ++u)
@@ -524,23 +524,17 @@ __device__ void afs_chunk(const AfsArgs& a, uint64_t c, int l, float* sw) {
             if (P >= (rsep ? kRowWords : kXRFeat / 2)) continue;
 #pragma unroll
             for (int q = 0; q < 4; q += 2)
-                *reinterpret_cast<float2*>(part + (hb + q) * 128 + 2 * P) =
-                    make_float2(fold_pair(s.d[2 * sb][q], s.d[2 * sb][q + 1]),
+                store_coherent2(part + (hb + q) * 128 + 2 * P, fold_pair(s.d[2 * sb][q], s.d[2 * sb][q + 1]),
                                 fold_pair(s.d[2 * sb + 1][q], s.d[2 * sb + 1][q + 1]));
         }
     }
     if (head && g == 0) {
-        part[kDenOff + n] = den;
-        part[kMOff + n] = s.m;
-        part[kMxOff + n] = s.mx;
+        store_coherent(part + kDenOff + n, den);
+        store_coherent(part + kMOff + n, s.m);
+        store_coherent(part + kMxOff + n, s.mx);
     }
     const uint32_t nch = uint32_t((rend - rbeg + a.chunk_edges - 1) / a.chunk_edges);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    uint32_t old = 0;
-    if (l == 0) old = __hip_atomic_fetch_add(a.counter + first, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    old = __shfl(old, 0);
-    if (old + 1 != nch) return;  // not the last chunk of this row
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (arrive(a.counter + first, l) + 1 != nch) return;  // not the last chunk of this row
     if (l == 0) a.counter[first] = 0;  // ready for the next launch
     afs_merge_row(a, first, l, sw);
 }

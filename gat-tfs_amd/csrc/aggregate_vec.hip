@@ -480,30 +480,25 @@ __device__ inline void run_chunk(const VArgs<ZT>& a, uint64_t c, int lane, int s
         for (int v = 0; v < C::VPL; ++v) {
             const int f0 = (sub + kWave * v) * C::VEC;
 #pragma unroll
-            for (int x = 0; x < C::VEC; x += 4)
-                *reinterpret_cast<float4*>(part + f0 + x) =
-                    make_float4(st.acc[v * C::VEC + x], st.acc[v * C::VEC + x + 1], st.acc[v * C::VEC + x + 2],
-                                st.acc[v * C::VEC + x + 3]);
+            for (int x = 0; x < C::VEC; x += 2)
+                store_coherent2(part + f0 + x, st.acc[v * C::VEC + x], st.acc[v * C::VEC + x + 1]);
             if (f0 % C::DIM == 0) {
-                part[C::W + st.h[v]] = st.den[v];
-                part[C::W + 8 + st.h[v]] = st.m[v];
+                store_coherent(part + C::W + st.h[v], st.den[v]);
+                store_coherent(part + C::W + 8 + st.h[v], st.m[v]);
             }
         }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    uint32_t old = 0;
-    if (lane == 0)
-        old = __hip_atomic_fetch_add(a.sp.counter + first, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    old = __shfl(old, 0);
-    if (old + 1 != nch) return;  // not the last chunk of this row
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (arrive(a.sp.counter + first, lane) + 1 != nch) return;  // not the last chunk of this row
     // Last arrival: the row max over the chunks, then the partials of every
-    // chunk in chunk order, scaled to it.
+    // chunk in chunk order, scaled to it, several chunks' loads in flight (one
+    // after the other, a row of 96 chunks was a chain of 192 round trips).
     float M[C::VPL];
 #pragma unroll
     for (int v = 0; v < C::VPL; ++v) {
         M[v] = -INFINITY;
-        for (uint32_t q = 0; q < nch; ++q) M[v] = fmaxf(M[v], a.sp.part[uint64_t(first + q) * PF + C::W + 8 + st.h[v]]);
+#pragma unroll 16
+        for (uint32_t q = 0; q < nch; ++q)
+            M[v] = fmaxf(M[v], load_coherent(a.sp.part + uint64_t(first + q) * PF + C::W + 8 + st.h[v]));
     }
     float tot[C::ACC];
     float dtot[C::VPL];
@@ -511,22 +506,21 @@ __device__ inline void run_chunk(const VArgs<ZT>& a, uint64_t c, int lane, int s
     for (int x = 0; x < C::ACC; ++x) tot[x] = 0.0f;
 #pragma unroll
     for (int v = 0; v < C::VPL; ++v) dtot[v] = 0.0f;
+#pragma unroll 4
     for (uint32_t q = 0; q < nch; ++q) {
         const float* pq = a.sp.part + uint64_t(first + q) * PF;
 #pragma unroll
         for (int v = 0; v < C::VPL; ++v) {
-            const float mq = pq[C::W + 8 + st.h[v]];
+            const float mq = load_coherent(pq + C::W + 8 + st.h[v]);
             const float f = mq == M[v] ? 1.0f : exp_w(mq - M[v]);  // a chunk of only -inf scores: 0
             const int f0 = (sub + kWave * v) * C::VEC;
 #pragma unroll
-            for (int x = 0; x < C::VEC; x += 4) {
-                const float4 t = *reinterpret_cast<const float4*>(pq + f0 + x);
+            for (int x = 0; x < C::VEC; x += 2) {
+                const float2 t = load_coherent2(pq + f0 + x);
                 tot[v * C::VEC + x] += t.x * f;
                 tot[v * C::VEC + x + 1] += t.y * f;
-                tot[v * C::VEC + x + 2] += t.z * f;
-                tot[v * C::VEC + x + 3] += t.w * f;
             }
-            dtot[v] += pq[C::W + st.h[v]] * f;
+            dtot[v] += load_coherent(pq + C::W + st.h[v]) * f;
         }
     }
     if (lane == 0) a.sp.counter[first] = 0;  // ready for the next launch

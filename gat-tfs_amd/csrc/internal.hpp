@@ -128,6 +128,38 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Partials of split rows, which waves of several XCDs write and one reads.  Each
+// XCD has an L2 of its own, and an agent-scope release fence writes all of it
+// back (an acquire invalidates it): thousands of chunks in flight paid for that
+// with the gather's cache (R-MAT 2^17 / 2M, 8 x 32: 180 us more for 128-edge
+// chunks than for 256).  So the partials alone bypass it: agent-scope relaxed
+// stores and loads (coherent over the device), a wait for the wave's own stores
+// before its arrival is counted, and loads that depend on the count read back.
+__device__ inline void store_coherent(float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void store_coherent2(float* p, float a, float b) {  // p 8-byte aligned
+    const uint64_t v = uint64_t(__builtin_bit_cast(uint32_t, b)) << 32 | __builtin_bit_cast(uint32_t, a);
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline float load_coherent(const float* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline float2 load_coherent2(const float* p) {  // p 8-byte aligned
+    const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float2(__builtin_bit_cast(float, uint32_t(v)), __builtin_bit_cast(float, uint32_t(v >> 32)));
+}
+// Counts the wave's arrival at `counter` once its coherent stores are done;
+// the count before it, in every lane.
+__device__ inline uint32_t arrive(uint32_t* counter, int lane) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint32_t old = 0;
+    if (lane == 0) old = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    old = __shfl(old, 0);
+    asm volatile("" ::: "memory");
+    return old;
+}
+
 // ---------------------------------------------------------------- launches
 // Every launcher returns hipSuccess or the launch error.
 
