@@ -86,11 +86,21 @@ struct LayerState {
 // 132 270) that gives 6144/2048 (8-head) and 4096/2048 (sum form, one head),
 // the best of measured sweeps there (sum form: 7.4 ms against 8.4 at
 // 8192/2048).
-enum { kPlanAf = 0, kPlanVec = 1, kPlanOne = 2, kPlans = 3 };
-constexpr uint32_t kPlanMin[kPlans] = {1024, 1536, 2048};
-constexpr uint32_t kPlanChunk[kPlans] = {256, 512, 1024};
-constexpr uint64_t kSmallGraphEdges = 16u << 20;
-constexpr uint32_t kSmallPlanMin = 512, kSmallPlanChunk = 256;
+//
+// Below kFineGraphEdges edges the transform-first launches do not fill the chip
+// and last as long as their longest chain of edges: chunks of 128 edges from
+// rows of 128 on (defaults only; the options apply as given).  Layer with 512/256
+// and with 128/128: 8 x 32, 30K rows / 450K edges 92 -> 66 us; 4 x 16 FP32,
+// 20K / 300K 45 -> 40.6; model on R-MAT 2^14 / 230K 149 -> 104; even at R-MAT
+// 2^16 / 900K (235 against 237), and 58 -> 61 us with one head at 1.2M edges,
+// where the partials' traffic is more than the chain.  kPlanCoarse keeps 512/256
+// for static layers whose scratch holds the fewer partials only.
+enum { kPlanAf = 0, kPlanVec = 1, kPlanOne = 2, kPlanCoarse = 3, kPlans = 4 };
+constexpr uint32_t kPlanMin[kPlans] = {1024, 1536, 2048, 0};
+constexpr uint32_t kPlanChunk[kPlans] = {256, 512, 1024, 0};
+constexpr uint64_t kSmallGraphEdges = 16u << 20, kFineGraphEdges = 1u << 20;
+constexpr uint32_t kSmallPlanMin = 512, kSmallPlanChunk = 256, kFinePlanMin = 128, kFinePlanChunk = 128;
+constexpr uint32_t kBlockMinDefault = 512;  // option GATGPU_OPT_BLOCK_ROW_MIN_DEGREE, unless set
 constexpr uint64_t kMaxChunksPerRow = 96;
 // Floats per split chunk in SplitTable::part: the widest partial row of the
 // transform-first kernels (512 features, 8 denominators, 8 chunk maxima).
@@ -121,6 +131,7 @@ struct TfBufs {
     bool keep_xbf = false;           // write the rounded input rows to xbf even when the convert is fused
     bool no_xbf = false;             // nobody reads the rounded input rows
     bool round_bf16 = false;         // out32 gets the widened values of bf16-stored rows
+    bool coarse = false;             // split rows by kPlanCoarse
     const uint32_t* out_perm = nullptr;  // one-head kernel: output row of sorted position k
     int ostride = 0;                     // its out32 row stride (floats)
     // The next layer's projection in this layer's aggregation epilogue
@@ -158,7 +169,9 @@ struct gatgpu_ctx {
     gatgpu::DevBuf xorig;  // the features in original node order (x32 is their sorted-order copy)
     gatgpu::LayerState L[3];
     // options (in-degree thresholds)
-    uint32_t block_min = 512;        // rows below this are never split
+    uint32_t block_min = gatgpu::kBlockMinDefault;  // rows below this are never split
+    bool block_min_set = false;      // by the user
+    bool fine_split = false;         // kPlanVec and kPlanOne split by kFinePlanMin, kPlanCoarse is built
     uint32_t split_min = 0;          // user option: rows >= this are split (0: per-kernel defaults)
     uint32_t split_chunk = 0;        // user option: edges per chunk (0: per-kernel defaults)
     bool keep_xbf = false;           // option GATGPU_OPT_KEEP_INPUT_BF16

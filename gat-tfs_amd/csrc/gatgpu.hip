@@ -74,20 +74,23 @@ int compute_bins(gatgpu_ctx* c) {
     uint32_t maxdeg = 0;  // degrees are sorted ascending
     if (c->n) HIPCHECK(c, hipMemcpy(&maxdeg, c->sorted_deg + (c->n - 1), 4, hipMemcpyDeviceToHost));
     const bool small = c->e < kSmallGraphEdges;
+    c->fine_split = c->e < kFineGraphEdges && !c->block_min_set && !c->split_min && !c->split_chunk;
+    const auto fine = [&](int q) { return c->fine_split && (q == kPlanVec || q == kPlanOne); };
     for (int q = 0; q < kPlans; ++q) {
         SplitPlan& P = c->plans[q];
-        const uint32_t min0 = small ? kSmallPlanMin : kPlanMin[q], chunk0 = small ? kSmallPlanChunk : kPlanChunk[q];
+        uint32_t min0 = small ? kSmallPlanMin : kPlanMin[q], chunk0 = small ? kSmallPlanChunk : kPlanChunk[q];
+        if (fine(q)) min0 = kFinePlanMin, chunk0 = kFinePlanChunk;
         uint32_t f = 1;
-        while (uint64_t(chunk0) * f * kMaxChunksPerRow < maxdeg && f < (1u << 12)) f *= 2;
-        const uint32_t min_scaled = q == kPlanVec ? min0 * f : std::max(min0, 2 * chunk0 * f);
+        while (chunk0 && uint64_t(chunk0) * f * kMaxChunksPerRow < maxdeg && f < (1u << 12)) f *= 2;
+        const uint32_t min_scaled = q == kPlanVec || fine(q) ? min0 * f : std::max(min0, 2 * chunk0 * f);
         P.min = c->split_min ? c->split_min : min_scaled;
         P.chunk = c->split_chunk ? c->split_chunk : chunk0 * f;
         thr[1 + q] = P.min - 1;
     }
     HIPCHECK(c, c->small.ensure(128));
-    // small[]: [0,4) max degree, [8,16) neighbor steps, [16,40) thresholds, [40,88) positions
+    // small[]: [0,4) max degree, [8,16) neighbor steps, [16,44) thresholds, [48,104) positions
     uint32_t* dthr = reinterpret_cast<uint32_t*>(c->small.as<char>() + 16);
-    uint64_t* dpos = reinterpret_cast<uint64_t*>(c->small.as<char>() + 40);
+    uint64_t* dpos = reinterpret_cast<uint64_t*>(c->small.as<char>() + 48);
     HIPCHECK(c, hipMemcpyAsync(dthr, thr, sizeof(thr), hipMemcpyHostToDevice, c->stream));
     HIPCHECK(c, launch_count_le(c->sorted_deg, c->n, dthr, 3 + kPlans, dpos, c->stream));
     uint64_t pos[3 + kPlans];
@@ -103,7 +106,11 @@ int compute_bins(gatgpu_ctx* c) {
     for (int q = 0; q < kPlans; ++q) {
         SplitPlan& P = c->plans[q];
         P.bins = b;
-        P.bins.split_begin = pos[1 + q] < b.block_begin ? b.block_begin : pos[1 + q];
+        P.bins.split_begin = pos[1 + q] < b.block_begin && !fine(q) ? b.block_begin : pos[1 + q];
+        if (q == kPlanCoarse && !c->fine_split) {  // nobody takes it
+            P.table = SplitTable{};
+            continue;
+        }
         // Chunk table of the split rows, heaviest row first.
         const uint64_t split_begin = P.bins.split_begin;
         const uint64_t nsplit = b.n - split_begin;
@@ -718,7 +725,7 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
     if (done) done->out_perm_used = a.out_perm != nullptr;
     // The row-group kernel takes its own split plan; the 8-head and fixed-p
     // kernels the 8-head one.
-    const SplitPlan& P = c->plans[grouped ? kPlanOne : kPlanVec];
+    const SplitPlan& P = c->plans[b.coarse ? kPlanCoarse : grouped ? kPlanOne : kPlanVec];
     SplitTable t = P.table;
     if (b.mchunk) t.mchunk = b.mchunk;
     if (b.part) t.part = b.part;
@@ -1227,7 +1234,10 @@ int gatgpu_set_option(gatgpu_ctx* c, int key, int64_t value) {
     if (int r = check_ctx(c)) return r;
     if (value < 0 || value > int64_t(UINT32_MAX)) return fail(c, GATGPU_EINVAL, "option value out of range");
     switch (key) {
-        case GATGPU_OPT_BLOCK_ROW_MIN_DEGREE: c->block_min = uint32_t(value); break;
+        case GATGPU_OPT_BLOCK_ROW_MIN_DEGREE:
+            c->block_min = uint32_t(value);
+            c->block_min_set = true;
+            break;
         case GATGPU_OPT_SPLIT_ROW_MIN_DEGREE:  // 0: the per-kernel defaults
             c->split_min = uint32_t(value);
             break;

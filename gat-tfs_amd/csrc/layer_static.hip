@@ -33,7 +33,7 @@ __global__ void k_fill_u32(uint32_t* p, uint64_t count, uint32_t v) {
 struct StaticPlan {
     uint64_t xbf = 0, z = 0, left = 0, right = 0, mx = 0, den = 0, out = 0, mchunk = 0, part = 0, counter = 0;
     uint64_t chunks = 0, bytes = 0;
-    bool outbf = false;
+    bool outbf = false, coarse = false;
 };
 
 uint64_t take(uint64_t& at, uint64_t bytes) {
@@ -42,7 +42,7 @@ uint64_t take(uint64_t& at, uint64_t bytes) {
     return off;
 }
 
-StaticPlan plan_static(const gatgpu_ctx* c, int layer, int precision, bool hidden) {
+StaticPlan plan_with(const gatgpu_ctx* c, int layer, int precision, bool hidden, bool coarse) {
     using namespace gatgpu;
     const LayerState& Ls = c->L[layer];
     const uint64_t n = c->n, K = uint64_t(Ls.heads), W = uint64_t(Ls.width());
@@ -59,12 +59,21 @@ StaticPlan plan_static(const gatgpu_ctx* c, int layer, int precision, bool hidde
     p.outbf = bf16 && hidden;
     p.out = take(at, p.outbf ? n * W * 2 : (n * W + kF32Pad) * 4);
     // Split rows of the 8-head and the one-head kernels' plans (whichever runs).
-    p.chunks = std::max(c->plans[kPlanVec].table.chunks, c->plans[kPlanOne].table.chunks);
+    p.coarse = coarse;
+    p.chunks = coarse ? c->plans[kPlanCoarse].table.chunks
+                      : std::max(c->plans[kPlanVec].table.chunks, c->plans[kPlanOne].table.chunks);
     p.mchunk = take(at, p.chunks * 8 * 4);
     p.part = take(at, p.chunks * kTfPartFloats * 4);
     p.counter = take(at, p.chunks * 4);
     p.bytes = at;
     return p;
+}
+
+// A small graph's short chunks need more partials than its coarse ones: where
+// only those fit the array, the layer takes them.
+StaticPlan plan_static(const gatgpu_ctx* c, int layer, int precision, bool hidden) {
+    const StaticPlan p = plan_with(c, layer, precision, hidden, false);
+    return p.bytes > kScratchBytes && c->fine_split ? plan_with(c, layer, precision, hidden, true) : p;
 }
 
 int check_static_args(gatgpu_ctx* c, int layer, int precision) {
@@ -136,6 +145,7 @@ int gatgpu_layer_forward_static(gatgpu_ctx* c, int layer, int precision, int hid
     b.outbf = !direct && p.outbf ? reinterpret_cast<uint16_t*>(base + p.out) : nullptr;
     b.round_bf16 = direct && p.outbf;
     b.no_xbf = true;
+    b.coarse = p.coarse;
     b.mchunk = reinterpret_cast<float*>(base + p.mchunk);
     b.part = reinterpret_cast<float*>(base + p.part);
     b.counter = reinterpret_cast<uint32_t*>(base + p.counter);

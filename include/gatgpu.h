@@ -116,11 +116,16 @@ typedef struct gatgpu_times {
 /* Options (gatgpu_set_option).  Thresholds are in-degrees. */
 enum {
     GATGPU_OPT_BLOCK_ROW_MIN_DEGREE = 1, /* rows below are never split (default
-                                            512; 0: no such limit)           */
+                                            512, or 128 on graphs below 1M
+                                            edges as long as options 1 to 3
+                                            are at their defaults; 0: no such
+                                            limit)                           */
     GATGPU_OPT_SPLIT_ROW_MIN_DEGREE = 2, /* rows at/above are split over waves
                                             (default per kernel: 1024 sum form,
                                             1536 8-head, 2048 one-head; 512 on
-                                            graphs below 16M edges; chunks
+                                            graphs below 16M edges, 128 in the
+                                            8-head and one-head kernels below
+                                            1M with the defaults; chunks
                                             doubled until the heaviest row has
                                             <= 96 of them, the degree with them
                                             (8-head) or at least 2 chunks (the
@@ -128,7 +133,8 @@ enum {
                                             0 restores them)                  */
     GATGPU_OPT_SPLIT_CHUNK_EDGES = 3,    /* edges per split chunk (default per
                                             kernel: 256, 512, 1024; 256 below
-                                            16M edges; scaled as above; a value
+                                            16M edges, 128 where rows of 128
+                                            are split; scaled as above; a value
                                             >= 64 applies to all, 0 restores) */
     /* 4 is not a key: rows of small degree take one wave each like the rest
        (or share one with rows of equal degree, where a row needs fewer lanes). */
@@ -281,7 +287,9 @@ int gatgpu_get_static_times(gatgpu_ctx* ctx, gatgpu_static_times* out);
  * which do allocate).  The work is enqueued on the context's stream
  * (gatgpu_stream) and the call returns without waiting; the stages of the
  * context are not touched.  Rejects (GATGPU_EOVERFLOW, before any launch) a
- * layer whose intermediates exceed the array.  Every call on one GPU shares
+ * layer whose intermediates exceed the array.  (On a graph below 1M edges a
+ * layer that fits only with the 512-edge split takes that: the same values up
+ * to the order of the sums.)  Every call on one GPU shares
  * that GPU's array: calls that overlap on one GPU (several contexts or host
  * threads, or streams not ordered against each other) race. */
 #define GATGPU_STATIC_SCRATCH_BYTES (64u << 20)
