@@ -493,7 +493,7 @@ __device__ void afs_merge_row(const AfsArgs& a, uint64_t c, int l, float* sw) {
 // Chunk c of a split row, one wave: sums against maxima of its own (the lazy
 // reference max and the exact max) into part[c][h * 128 + f], the
 // denominators and both maxima after them; the last chunk of the row to
-// arrive (agent-scope release/acquire around a relaxed counter) merges the
+// arrive (coherent partials and a relaxed counter, internal.hpp) merges the
 // row.  sw: the wave's kMergeFloats of LDS.
 __device__ void afs_chunk(const AfsArgs& a, uint64_t c, int l, float* sw) {
     const int g = l / 16, n = l % 16;

@@ -8,7 +8,7 @@
 //   * chunks of split rows (in-degree >= split_min), C edges each.  A chunk
 //     runs the online softmax over its edges as a whole row does and leaves
 //     its partial (sum p Z, sum p) with its own max m_c in scratch; the last
-//     chunk to arrive (agent-scope release/acquire around a relaxed counter)
+//     chunk to arrive (coherent partials and a relaxed counter, internal.hpp)
 //     scales each partial by e^(m_c - M), M the row max, adds them in chunk
 //     order, which is deterministic, and finishes the row.
 //   * whole rows below split_min, heaviest first.
@@ -30,8 +30,7 @@
 // running-maximum form of implementation/src/gat_tfs_online.cpp:86-117).  Each
 // edge slot keeps its own state and the slots merge at the end of the row.
 // Every source row is thus read once, and the final m is max leaky(L + R_j) =
-// leaky(L + max R_j) bit for bit (leaky and the addition are monotone).  A
-// chunk starts from the exact row max, so its m never moves.
+// leaky(L + max R_j) bit for bit (leaky and the addition are monotone).
 #include "internal.hpp"
 
 namespace gatgpu {
