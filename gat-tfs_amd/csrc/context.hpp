@@ -133,6 +133,7 @@ struct TfBufs {
     bool no_xbf = false;             // nobody reads the rounded input rows
     bool round_bf16 = false;         // out32 gets the widened values of bf16-stored rows
     bool coarse = false;             // split rows by kPlanCoarse
+    uint64_t clear = 0;              // counters to zero before the aggregation: by the projection where it can
     const uint32_t* out_perm = nullptr;  // one-head kernel: output row of sorted position k
     int ostride = 0;                     // its out32 row stride (floats)
     // The next layer's projection in this layer's aggregation epilogue

@@ -661,6 +661,13 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
     // kept (stage XBF).
     const bool keep_xbf = b.keep_xbf || (!in_loads && !b.no_xbf);
     if (done) done->fused_convert = fused && !keep_xbf;
+    // The static layer's counters, in the projection's launch where it takes them.
+    if (b.clear && tile) {
+        pa.clear = b.counter;
+        pa.nclear = b.clear;
+    } else if (b.clear && !(!bf16 && Ls.wpk32.p)) {
+        HIPCHECK(c, launch_clear_u32(b.counter, b.clear, c->stream));
+    }
     if (b.projected) {
         // Z, L and R come from the previous layer's epilogue: no convert, no projection.
     } else if (bf16 && src32 && !fused) {
@@ -703,6 +710,10 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
         fa.left = b.left;
         fa.right = b.right;
         fa.tiles = (n + 31) / 32;
+        if (b.clear) {
+            fa.clear = b.counter;
+            fa.nclear = b.clear;
+        }
         HIPCHECK(c, launch_projection_split(fa, c->stream, c->cus));
     } else {
         HIPCHECK(c, launch_projection(src32, nullptr, Ls.w32.as<float>(), n, D, K, dim, Ls.al.as<float>(),

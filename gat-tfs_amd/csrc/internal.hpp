@@ -160,6 +160,13 @@ __device__ inline uint32_t arrive(uint32_t* counter, int lane) {
     return old;
 }
 
+// Words [0, count) to zero by the whole grid, for a later launch.
+__device__ inline void clear_words(uint32_t* p, uint64_t count) {
+    if (!p) return;
+    for (uint64_t i = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; i < count; i += uint64_t(gridDim.x) * blockDim.x)
+        p[i] = 0;
+}
+
 // ---------------------------------------------------------------- launches
 // Every launcher returns hipSuccess or the launch error.
 
@@ -194,6 +201,7 @@ hipError_t launch_gather_rows(const void* src, uint64_t src_stride_words, void* 
 // Rows of `width` floats at stride `stride` to dense rows; dst (16-byte aligned)
 // may be host memory mapped to the device.
 hipError_t launch_pack_rows(const float* src, uint64_t stride, float* dst, uint64_t rows, uint32_t width, hipStream_t s);
+hipError_t launch_clear_u32(uint32_t* p, uint64_t count, hipStream_t s);
 hipError_t launch_count_le(const uint32_t* sorted_deg, uint64_t n, const uint32_t* thresholds,
                            int count, uint64_t* positions, hipStream_t s);
 
@@ -234,6 +242,8 @@ struct ProjArgs {
     int xouts;           // rows, features [0, 16 ksteps), at xout[row * xouts]
     bool r_from_z;       // bf16 8 x 32 or one head x 64: R = Z_bf16 . aR (the aggregation recomputes it)
     const float* ar;     // aR [256] when r_from_z
+    uint32_t* clear;     // words [0, nclear) to zero on the way (the projections that
+    uint64_t nclear;     // take them: launch_projection_tile), or null
     const float* al;     // aL [heads * dim]: the W-stationary path forms L and R from FP32 Z
 };
 // R from the stored bf16 Z: the fast projection writes R = Z_bf16 . aR and
@@ -275,6 +285,8 @@ struct ProjF32Args {
     float* left;         // [n][heads]
     float* right;        // [n][heads]
     uint64_t tiles;      // ceil(n / 32)
+    uint32_t* clear;     // words [0, nclear) to zero on the way, or null
+    uint64_t nclear;
     // set by the launch: the k range and output blocks of one kernel launch
     int k0, kn, nob;
     bool add;

@@ -75,6 +75,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     __shared__ __attribute__((aligned(16))) uint2 xs[2][U][3][2 * kWave];
     __shared__ float plr[2][kWaves][2][32];       // L and R shares of a wave's rows, two tiles
     __shared__ float alr[2][kWaves][32];          // aL, aR of the group's output blocks
+    clear_words(a.clear, a.nclear);
     __shared__ int bad[3];
     // Beyond 128 inputs the third parts of W (one of the six terms) stay in LDS:
     // 12 KS registers would not leave room for the rest.

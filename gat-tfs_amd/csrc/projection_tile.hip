@@ -31,6 +31,7 @@ __global__ void __launch_bounds__((KS > 16 ? 8 : 9) * kWave) k_proj_tile(ProjArg
     const int nb = a.head_blocks + 1, ks_n = a.ksteps;
     const int tl = w / nb, ob = w % nb;
     const bool lr = ob == a.head_blocks, act = tl < tpb;
+    clear_words(a.clear, a.nclear);
     uint4 wf[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)

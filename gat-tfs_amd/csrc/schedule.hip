@@ -331,6 +331,8 @@ __global__ void k_count_le(const uint32_t* __restrict__ sorted_deg, uint64_t n,
     pos[q] = lo;
 }
 
+__global__ void k_clear_u32(uint32_t* p, uint64_t count) { clear_words(p, count); }
+
 uint32_t grid_for(uint64_t items, uint64_t per_block, uint32_t cap) {
     uint64_t g = (items + per_block - 1) / per_block;
     if (g < 1) g = 1;
@@ -424,6 +426,12 @@ hipError_t launch_pack_rows(const float* src, uint64_t stride, float* dst, uint6
     if (!rows) return hipSuccess;
     k_pack_rows<<<grid_for((rows + kPackRows - 1) / kPackRows, 1, 2048), kThreads, 0, s>>>(src, stride, dst, rows,
                                                                                          width);
+    return hipGetLastError();
+}
+
+hipError_t launch_clear_u32(uint32_t* p, uint64_t count, hipStream_t s) {
+    if (!count) return hipSuccess;
+    k_clear_u32<<<dim3(grid_for(count, 256, 1024)), 256, 0, s>>>(p, count);
     return hipGetLastError();
 }
 
