@@ -46,7 +46,6 @@ struct LayerState {
     DevBuf z32, zbf, left, right, mx, den, out32, outbf, in32, inbf;
     // What the last forward of this layer produced.
     bool ran = false, z_valid = false, out32_valid = false, outbf_valid = false;
-    bool z_deferred = false;    // aggregate-first by the edge rule: stage Z is projected from inbf when asked for
     bool out_original = false;  // out32 rows in original node order (else sorted order)
     int out_stride = 0;         // out32 row stride (floats): the width, or k1_out_stride when out_original
     bool xbf_valid = false;     // inbf holds the rounded layer input rows

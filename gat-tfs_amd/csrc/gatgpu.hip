@@ -223,21 +223,6 @@ int resolve_dataflow(const LayerState& L, int precision, int dataflow, uint64_t 
     return dataflow;
 }
 
-// The model's first layer also takes the sum form below kAfMinZBytes from this many
-// edges on: it moves 256 bytes an edge instead of 512 or 1024, against tiles that
-// wait for their heaviest rows and a fetch of R beside the row beyond 112
-// inputs.  Transform-first against sum form, us of the whole model (R-MAT is the
-// least favourable family, its heavy rows last longest):
-//   8 x 32, 100 inputs: 240K nodes / 9.6M edges 1766 / 1427, 480K / 7.2M 1674 /
-//   1454, 360K / 9M 2980 / 2690; R-MAT 2^17 / 5M 663 / 676, 240K / 1.4M 581 / 584;
-//   8 x 32, 128 inputs: 240K / 9.6M 1755 / 1543; R-MAT 2^17 / 5M 671 / 723;
-//   8 x 64, 100 inputs: 120K / 1.8M 858 / 642, R-MAT 2^17 / 2M 748 / 661; 2^16 / 1M 395 / 391;
-//   8 x 64, 128 inputs: 240K / 3.6M 1598 / 1213; R-MAT 2^17 / 2M 700 / 703.
-uint64_t sum_form_min_edges(const LayerState& L) {
-    if (L.dim == 64) return L.in <= kXRFeat ? 1500000 : 2500000;
-    return L.in <= kXRFeat ? 6000000 : 8000000;
-}
-
 float ms_between(hipEvent_t a, hipEvent_t b) {
     float ms = 0.0f;
     if (hipEventElapsedTime(&ms, a, b) != hipSuccess) return 0.0f;
@@ -431,7 +416,7 @@ int run_layer_af(gatgpu_ctx* c, int l, bool hidden, const float* src32, const ui
     Ls.ran = true;
     Ls.precision = GATGPU_BF16;
     Ls.dataflow = dataflow;
-    Ls.z_valid = Ls.z_deferred = false;
+    Ls.z_valid = false;
     Ls.out32_valid = !hidden;
     Ls.outbf_valid = hidden;
     return GATGPU_OK;
@@ -602,7 +587,6 @@ int run_layer(gatgpu_ctx* c, int l, int precision, int dataflow, bool hidden, co
     Ls.precision = precision;
     Ls.dataflow = GATGPU_TRANSFORM_FIRST;
     Ls.z_valid = true;
-    Ls.z_deferred = false;
     // With the next projection fused, only the split rows store their output.
     Ls.out32_valid = !want_outbf;
     Ls.outbf_valid = want_outbf && fuse != kFuseNext;
@@ -798,37 +782,6 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
 }  // namespace gatgpu
 
 namespace {
-
-// Z of a layer the edge rule ran aggregate-first, from its rounded input rows: the
-// rows transform-first would have stored.  L and R of this projection go to a
-// buffer of no stage (the layer's own are the aggregation's).
-int project_deferred(gatgpu_ctx* c, int l) {
-    LayerState& Ls = c->L[l];
-    const uint64_t n = c->n, K = uint64_t(Ls.heads);
-    HIPCHECK(c, hipSetDevice(c->device));
-    ProjArgs pa{};
-    pa.zs = z_stride(GATGPU_BF16, Ls.heads, Ls.width(), nullptr);
-    HIPCHECK(c, Ls.zbf.ensure(n * uint64_t(pa.zs) * 2));
-    HIPCHECK(c, Ls.in32.ensure(2 * n * K * 4));
-    pa.n = n;
-    pa.x = Ls.inbf.as<uint16_t>();
-    pa.xs = Ls.xbf_stride;
-    pa.ksteps = Ls.ksteps;
-    pa.wpk = Ls.wpk.as<uint4>();
-    pa.groups = Ls.groups;
-    pa.head_blocks = (Ls.width() + 31) / 32;
-    pa.nmb = Ls.nmb;
-    pa.width = Ls.width();
-    pa.heads = Ls.heads;
-    pa.z = Ls.zbf.as<uint16_t>();
-    pa.left = Ls.in32.as<float>();
-    pa.right = pa.left + n * K;
-    pa.tiles = (n + 31) / 32;
-    HIPCHECK(c, launch_projection_mfma(pa, c->stream, c->cus));
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    Ls.z_valid = true;
-    return GATGPU_OK;
-}
 
 void fill_times(gatgpu_ctx* c, int ev_base, gatgpu_times* t, int dataflow) {
     std::memset(t, 0, sizeof(*t));
@@ -1162,10 +1115,6 @@ int gatgpu_model_forward(gatgpu_ctx* c, int precision, int dataflow, float* logi
         flows[l] = resolve_dataflow(c->L[l], precision, dataflow, c->n);
         if (flows[l] < 0) flows[l] = GATGPU_TRANSFORM_FIRST;
     }
-    const bool by_edges = dataflow == GATGPU_AUTO && precision == GATGPU_BF16 && flows[0] == GATGPU_TRANSFORM_FIRST &&
-                          aggregate_afsum_supported(c->L[0].in, c->L[0].heads, c->L[0].dim, c->n) &&
-                          c->e >= sum_form_min_edges(c->L[0]);
-    if (by_edges) flows[0] = GATGPU_AGGREGATE_FIRST;
     // Option 1 fuses on graphs of at least kSmallGraphEdges edges only.  On
     // smaller graphs each 32-row tile's waves aggregate their rows one after
     // another, and the tiles of the heaviest unsplit rows outlast the rest of
@@ -1178,7 +1127,6 @@ int gatgpu_model_forward(gatgpu_ctx* c, int precision, int dataflow, float* logi
         const int fuse = !fuse23 ? kFuseNone : l == 1 ? kFuseNext : l == 2 ? kProjected : kFuseNone;
         if (int r = run_layer(c, l, precision, flows[l], l < 2, nullptr, stages ? 4 * l : -1, false, l == 2, fuse))
             return r;
-        if (l == 0) c->L[0].z_deferred = by_edges;
     }
     // Logits in original node order, inside the timed forward: written so by
     // the last aggregation where it can, else gathered back (row i = sorted
@@ -1224,7 +1172,7 @@ int gatgpu_stage_size(gatgpu_ctx* c, int layer, int which, uint64_t* count) {
     if (!L.ran) return GATGPU_OK;
     switch (which) {
         case GATGPU_STAGE_Z:
-            *count = L.z_valid || L.z_deferred ? c->n * L.width() : 0;
+            *count = L.z_valid ? c->n * L.width() : 0;
             break;
         case GATGPU_STAGE_LEFT:
         case GATGPU_STAGE_RIGHT:
@@ -1249,8 +1197,6 @@ int gatgpu_get_stage(gatgpu_ctx* c, int layer, int which, float* host) {
     if (int r = gatgpu_stage_size(c, layer, which, &count)) return r;
     if (!count) return fail(c, GATGPU_ESTATE, "stage not available");
     if (!host) return fail(c, GATGPU_EINVAL, "null output");
-    if (which == GATGPU_STAGE_Z && !c->L[layer].z_valid)
-        if (int r = project_deferred(c, layer)) return r;
     const LayerState& L = c->L[layer];
     const void* src = nullptr;
     bool bf = false;

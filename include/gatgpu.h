@@ -69,10 +69,7 @@ enum { GATGPU_FP32 = 0, GATGPU_BF16 = 1 };
  * and p (X_j W_h) summed, in the neighbour-step order of
  * baseline/src/baseline_tfs.cpp:16-110.  AUTO selects the sum form where it
  * applies (bf16) and the layer's bf16 Z table (n x heads x head_dim x 2 bytes)
- * exceeds 256 MB, and transform-first elsewhere; gatgpu_model_forward also
- * takes it for its first layer on graphs of many edges (from 1.5M to 8M, by
- * head_dim and in), whose stage Z gatgpu_get_stage then projects when asked.
- * gatgpu_model_forward with
+ * exceeds 256 MB, and transform-first elsewhere.  gatgpu_model_forward with
  * AGGREGATE_FIRST uses it on the layers that support it and transform-first
  * on the others. */
 /* TFS_B1 is the faithful neighbour-step TFS ("tfs_bf16",
