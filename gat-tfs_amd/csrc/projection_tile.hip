@@ -139,9 +139,17 @@ __global__ void __launch_bounds__((KS > 16 ? 8 : 9) * kWave) k_proj_tile(ProjArg
 #pragma unroll
                 for (int q8 = 0; q8 < 2; ++q8) {
                     const int f0 = 32 * ob + 16 * half + 8 * q8;
-                    if (ok && f0 < a.width)
-                        *reinterpret_cast<uint4*>(a.z + row * a.zs + f0) =
+                    uint16_t* to = a.z + row * a.zs + f0;
+                    if (ok && f0 < a.width && !(a.r_in_z && f0 + 8 > a.r_off)) {
+                        *reinterpret_cast<uint4*>(to) =
                             make_uint4(zp[4 * q8], zp[4 * q8 + 1], zp[4 * q8 + 2], zp[4 * q8 + 3]);
+                    } else if (ok && f0 < a.width) {
+                        // The piece that ends in R (57 to 60 features): the L/R
+                        // block's wave writes those four bytes, in no order with
+                        // this one, so they are left alone here.
+                        *reinterpret_cast<uint2*>(to) = make_uint2(zp[4 * q8], zp[4 * q8 + 1]);
+                        *reinterpret_cast<uint32_t*>(to + 4) = zp[4 * q8 + 2];
+                    }
                 }
                 if (a.r_from_z) {
                     // R = Z_bf16 . aR in the aggregation's order: an FMA chain over
@@ -231,6 +239,8 @@ bool projection_tile_shape(const ProjArgs& a) {
 hipError_t launch_projection_tile(const ProjArgs& a, hipStream_t s, int cus) {
     if (!projection_tile_shape(a) || a.tiles != (a.n + 31) / 32 || (a.r_from_z && (!a.ar || a.heads != 8 || a.width != 256)))
         return hipErrorInvalidValue;
+    // R in the row: the last four bytes of its last 16-byte piece.
+    if (a.r_in_z && (a.heads != 1 || a.zs % 8 || a.r_off != a.zs - 2 || a.width > a.r_off)) return hipErrorInvalidValue;
     return a.x32 ? launch_ks<true>(a, s, cus) : launch_ks<false>(a, s, cus);
 }
 

@@ -73,3 +73,41 @@ def test_static_layer_unaligned_rows(gpu_ctx, D, K, d, hidden):
         outs.append(out[shift:shift + n * W].cpu().numpy())
         assert torch.isnan(torch.cat([out[:shift], out[shift + n * W:]])).all()
     assert np.all(np.isfinite(outs[0])) and np.array_equal(outs[0], outs[1])
+
+
+def check_r_in_rows(ctx, layer, col, n):
+    """Rows of one edge each: the row max is LeakyReLU(L + R) of the R the aggregation reads in its
+    source's Z row, so it carries that R's bits."""
+    left, right, top = (ctx.stage(layer, k).reshape(n) for k in ("left", "right", "max"))
+    s = left + right[col]
+    assert np.array_equal(np.maximum(s, np.float32(0.2) * s), top)
+
+
+@pytest.mark.parametrize("width", [1, 55, 56, 57, 58, 59, 60])
+@pytest.mark.parametrize("D,n", [(40, 33), (256, 1000), (100, 20_011), (512, 20_011), (200, 70_001)])
+def test_r_beside_the_last_features(gpu_ctx, width, D, n):
+    """One head whose Z rows end in R: the widths whose last 16-byte piece of features holds it, and
+    those just below, over partial tiles and 1 to 4 tiles a block."""
+    row, col = np.arange(n + 1, dtype=np.uint64), ((np.arange(n) * 7 + 1) % n).astype(np.uint32)
+    x = inputs.normal((n, D), D + n)
+    p = inputs.glorot_param(D, 1, width, 9)
+    gpu_ctx.set_graph(row, col)
+    gpu_ctx.set_layer(0, p)
+    gpu_ctx.set_input(x)
+    gpu_ctx.layer_forward(0, gatgpu.BF16, gatgpu.TRANSFORM_FIRST, False)
+    check_r_in_rows(gpu_ctx, 0, col, n)
+    # one edge a row: the output is the source's Z row
+    assert np.array_equal(gpu_ctx.stage(0, "out"), gpu_ctx.stage(0, "z")[col])
+
+
+@pytest.mark.parametrize("classes", [57, 60])
+def test_r_beside_the_last_features_from_bf16_rows(gpu_ctx, classes):
+    """The same for the output layer of a model, whose input rows are bf16 already."""
+    n = 20_011
+    row, col = np.arange(n + 1, dtype=np.uint64), ((np.arange(n) * 7 + 1) % n).astype(np.uint32)
+    gpu_ctx.set_graph(row, col)
+    gpu_ctx.set_model(inputs.glorot_model(64, 8, 32, classes, 4))
+    gpu_ctx.set_input(inputs.normal((n, 64), 5))
+    logits, _, _ = gpu_ctx.model_forward(gatgpu.BF16, gatgpu.TRANSFORM_FIRST)
+    check_r_in_rows(gpu_ctx, 2, col, n)
+    assert np.array_equal(logits, gpu_ctx.stage(2, "z")[col])
