@@ -23,7 +23,11 @@ typedef float f32x16 __attribute__((__vector_size__(16 * sizeof(float))));
 
 
 // KS: the most k steps (a.ksteps of them used).  tpb: tiles a block takes at once.
-template <int KS, bool F32IN>
+// TAIL: R lies in the 16 bytes of the row's last features (one head of 57 to 60):
+// the L/R block's wave writes R, in no order with the wave of those features, so
+// that one leaves the four bytes out.  (A template parameter: the test of a kernel
+// argument in the store cost 1.5 us a launch, in registers spilled.)
+template <int KS, bool F32IN, bool TAIL>
 __global__ void __launch_bounds__((KS > 16 ? 8 : 9) * kWave) k_proj_tile(ProjArgs a, int tpb) {
     extern __shared__ __attribute__((aligned(16))) uint4 xs[];  // [2][tpb][ksteps][64]
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave), l = threadIdx.x % kWave;
@@ -139,17 +143,15 @@ __global__ void __launch_bounds__((KS > 16 ? 8 : 9) * kWave) k_proj_tile(ProjArg
 #pragma unroll
                 for (int q8 = 0; q8 < 2; ++q8) {
                     const int f0 = 32 * ob + 16 * half + 8 * q8;
+                    if (!ok || f0 >= a.width) continue;
                     uint16_t* to = a.z + row * a.zs + f0;
-                    if (ok && f0 < a.width && !(a.r_in_z && f0 + 8 > a.r_off)) {
-                        *reinterpret_cast<uint4*>(to) =
-                            make_uint4(zp[4 * q8], zp[4 * q8 + 1], zp[4 * q8 + 2], zp[4 * q8 + 3]);
-                    } else if (ok && f0 < a.width) {
-                        // The piece that ends in R (57 to 60 features): the L/R
-                        // block's wave writes those four bytes, in no order with
-                        // this one, so they are left alone here.
+                    if (TAIL && f0 + 8 > a.r_off) {
                         *reinterpret_cast<uint2*>(to) = make_uint2(zp[4 * q8], zp[4 * q8 + 1]);
                         *reinterpret_cast<uint32_t*>(to + 4) = zp[4 * q8 + 2];
+                        continue;
                     }
+                    *reinterpret_cast<uint4*>(to) =
+                        make_uint4(zp[4 * q8], zp[4 * q8 + 1], zp[4 * q8 + 2], zp[4 * q8 + 3]);
                 }
                 if (a.r_from_z) {
                     // R = Z_bf16 . aR in the aggregation's order: an FMA chain over
@@ -195,7 +197,7 @@ __global__ void __launch_bounds__((KS > 16 ? 8 : 9) * kWave) k_proj_tile(ProjArg
 
 int tiles_per_block(int head_blocks) { return head_blocks == 1 ? 4 : head_blocks <= 3 ? 2 : 1; }
 
-template <int KS, bool F32IN>
+template <int KS, bool F32IN, bool TAIL>
 hipError_t launch(const ProjArgs& a, hipStream_t s, int cus) {
     // Few tiles: one a block, so that more CUs share them; and what fits LDS
     // beside the 1 KB of aR.
@@ -204,7 +206,7 @@ hipError_t launch(const ProjArgs& a, hipStream_t s, int cus) {
     while (tpb > 1 && ((a.tiles + tpb - 1) / tpb < uint64_t(cus) || bytes(tpb) > 128 * 1024)) tpb /= 2;
     const size_t lds = bytes(tpb);
     if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_proj_tile<KS, F32IN>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_proj_tile<KS, F32IN, TAIL>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess) return e;
     }
@@ -217,16 +219,16 @@ hipError_t launch(const ProjArgs& a, hipStream_t s, int cus) {
     uint64_t grid = uint64_t(cus) * per_cu;
     const uint64_t groups = (a.tiles + tpb - 1) / tpb;
     if (grid > groups) grid = groups;
-    k_proj_tile<KS, F32IN><<<dim3(uint32_t(grid)), threads, lds, s>>>(a, tpb);
+    k_proj_tile<KS, F32IN, TAIL><<<dim3(uint32_t(grid)), threads, lds, s>>>(a, tpb);
     return hipGetLastError();
 }
 
-template <bool F32IN>
+template <bool F32IN, bool TAIL>
 hipError_t launch_ks(const ProjArgs& a, hipStream_t s, int cus) {
-    if (a.ksteps <= 4) return launch<4, F32IN>(a, s, cus);
-    if (a.ksteps <= 8) return launch<8, F32IN>(a, s, cus);
-    if (a.ksteps <= 16) return launch<16, F32IN>(a, s, cus);
-    return launch<32, F32IN>(a, s, cus);
+    if (a.ksteps <= 4) return launch<4, F32IN, TAIL>(a, s, cus);
+    if (a.ksteps <= 8) return launch<8, F32IN, TAIL>(a, s, cus);
+    if (a.ksteps <= 16) return launch<16, F32IN, TAIL>(a, s, cus);
+    return launch<32, F32IN, TAIL>(a, s, cus);
 }
 
 }  // namespace
@@ -241,7 +243,8 @@ hipError_t launch_projection_tile(const ProjArgs& a, hipStream_t s, int cus) {
         return hipErrorInvalidValue;
     // R in the row: the last four bytes of its last 16-byte piece.
     if (a.r_in_z && (a.heads != 1 || a.zs % 8 || a.r_off != a.zs - 2 || a.width > a.r_off)) return hipErrorInvalidValue;
-    return a.x32 ? launch_ks<true>(a, s, cus) : launch_ks<false>(a, s, cus);
+    if (a.r_in_z && a.width > a.zs - 8) return a.x32 ? launch_ks<true, true>(a, s, cus) : launch_ks<false, true>(a, s, cus);
+    return a.x32 ? launch_ks<true, false>(a, s, cus) : launch_ks<false, false>(a, s, cus);
 }
 
 }  // namespace gatgpu
