@@ -164,9 +164,11 @@ struct Lane {
     }
 };
 
-// One batch of NB edges (the first cnt of them real; the others read row 0
-// with weight 0): all loads, then scores, the rescale and the sums.
-template <class C, int NB>
+// One batch of NB edges: all loads, then scores, the rescale and the sums.  Only
+// the first cnt of them (SURE at least) are real.  The others read the row's
+// last source again (the batch loads it anyway) and add 0 * 0, whatever it holds:
+// a weight of 0 alone would make NaN of an infinity.
+template <class C, int NB, int SURE>
 __device__ inline void batch(const GrpArgs<typename C::ZT>& a, Lane<C>& s, uint32_t j, int cnt) {
     using ZT = typename C::ZT;
     using Raw = typename C::Raw;
@@ -204,7 +206,7 @@ __device__ inline void batch(const GrpArgs<typename C::ZT>& a, Lane<C>& s, uint3
         }
 #pragma unroll
         for (int v = 0; v < C::VPL; ++v) {
-            r[t][v] = t < cnt ? leaky(s.Li[v] + r[t][v]) : -INFINITY;
+            r[t][v] = t < SURE || t < cnt ? leaky(s.Li[v] + r[t][v]) : -INFINITY;
             mb[v] = fmaxf(mb[v], r[t][v]);
         }
     }
@@ -231,10 +233,11 @@ __device__ inline void batch(const GrpArgs<typename C::ZT>& a, Lane<C>& s, uint3
     for (int t = 0; t < NB; ++t) {
 #pragma unroll
         for (int v = 0; v < C::VPL; ++v) {
-            const float p = t < cnt ? exp_w(r[t][v] - s.m[v]) : 0.0f;
+            const bool real = t < SURE || t < cnt;
+            const float p = real ? exp_w(r[t][v] - s.m[v]) : 0.0f;
             s.d[v] += p;
             float f[C::VEC];
-            unpack<ZT, C::VEC>(raw[t][v], f);
+            unpack<ZT, C::VEC>(real ? raw[t][v] : Raw{}, f);
 #pragma unroll
             for (int x = 0; x < C::VEC; ++x) s.acc[v][x] += p * f[x];
         }
@@ -255,12 +258,12 @@ __device__ inline void edges(const GrpArgs<typename C::ZT>& a, Lane<C>& s, uint6
     for (uint32_t done = start; done < total; done += step) {
         const uint32_t left = total - done;
         const int cnt = left < uint32_t(C::B) ? int(left) : C::B;
-        const uint32_t j = s.sub < cnt ? next : 0u;
+        const uint32_t j = next;  // past the end: the last source
         next = id_at(done + step + lane_t);
         // Half a batch's loads where half hold the rest of the row: most rows
         // of a skewed graph have a few edges only.
-        if (left > uint32_t(C::B) / 2) batch<C, C::B>(a, s, j, cnt);
-        else batch<C, C::B / 2>(a, s, j, cnt);
+        if (left > uint32_t(C::B) / 2) batch<C, C::B, C::B / 2 + 1>(a, s, j, cnt);
+        else batch<C, C::B / 2, 1>(a, s, j, cnt);
     }
 }
 
