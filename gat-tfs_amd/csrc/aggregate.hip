@@ -20,6 +20,7 @@
 // are rescaled when a batch raises m (the running-maximum form of
 // implementation/src/gat_tfs_online.cpp:86-117); the final m equals
 // leaky(L + max R) bit for bit, because leaky and the addition are monotone.
+// Scores of -inf weigh 0 as soon as the row has a finite one.
 //
 // Bound: misses in flight times latency, and for rows of many edges the chain
 // of batches.  So rows are split by degree (sorted, heaviest first), all in
@@ -43,6 +44,10 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWavesPerBlock = kThreads / kWave;
+// A row's maximum before its first edge: finite, so that scores of -inf weigh
+// exp(-inf - kNoMax) = 0 while nothing else was met (from -inf they would weigh
+// exp(-inf + inf), NaN, and with them the row).
+constexpr float kNoMax = -3.402823466e38f;
 constexpr uint32_t kPartStride = 512 + 16;  // sums, denominators of the heads, maxima of the heads
 
 template <int BYTES>
@@ -156,7 +161,7 @@ struct Lane {
 #pragma unroll
         for (int v = 0; v < C::VPL; ++v) {
             Li[v] = a.L[uint64_t(i) * a.K + head[v]];
-            m[v] = -INFINITY;
+            m[v] = kNoMax;
             d[v] = 0.0f;
 #pragma unroll
             for (int x = 0; x < C::VEC; ++x) acc[v][x] = 0.0f;
@@ -223,7 +228,7 @@ __device__ inline void batch(const GrpArgs<typename C::ZT>& a, Lane<C>& s, uint3
 #pragma unroll
     for (int v = 0; v < C::VPL; ++v) {
         const float mn = fmaxf(s.m[v], mb[v]);
-        const float sc = exp_w(s.m[v] - mn);  // 0 on the first batch (m = -inf)
+        const float sc = exp_w(s.m[v] - mn);  // 0 on the first batch (m = kNoMax)
         s.m[v] = mn;
         s.d[v] *= sc;
 #pragma unroll
@@ -268,7 +273,7 @@ __device__ inline void edges(const GrpArgs<typename C::ZT>& a, Lane<C>& s, uint6
 }
 
 // Partials of the wave's groups into every group: m to the common maximum, the
-// sums scaled to it and added.  Groups without edges (m = -inf, sums 0) add 0.
+// sums scaled to it and added.  Groups without edges (m = kNoMax, sums 0) add 0.
 template <class C>
 __device__ inline void merge_groups(Lane<C>& s) {
 #pragma unroll
@@ -293,11 +298,14 @@ __device__ inline void finish(const GrpArgs<typename C::ZT>& a, const Lane<C>& s
     constexpr int V = C::VEC;
 #pragma unroll
     for (int v = 0; v < C::VPL; ++v) {
+        // Nothing but scores of -inf (or NaN): no softmax, as exp(-inf - max) is NaN.
+        const bool none = any && s.m[v] == kNoMax && !(s.d[v] > 0.0f);
+        const float d = none ? NAN : s.d[v];
         if (s.lead[v]) {
-            a.mx[uint64_t(i) * a.K + s.head[v]] = any ? s.m[v] : 0.0f;
-            a.den[uint64_t(i) * a.K + s.head[v]] = s.d[v];
+            a.mx[uint64_t(i) * a.K + s.head[v]] = none ? -INFINITY : any ? s.m[v] : 0.0f;
+            a.den[uint64_t(i) * a.K + s.head[v]] = d;
         }
-        const float scale = s.d[v] > 0.0f ? 1.0f / s.d[v] : 0.0f;
+        const float scale = none ? NAN : d > 0.0f ? 1.0f / d : 0.0f;
         float y[V];
 #pragma unroll
         for (int x = 0; x < V; ++x) {

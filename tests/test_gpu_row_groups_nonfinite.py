@@ -3,7 +3,8 @@
 A batch's lanes past the row's last edge must not carry
 another row's infinity or NaN into a row that is not connected to it; a row
 connected to an infinite Z entry has that entry infinite, whatever the position
-of the edge.
+of the edge; and edges with a score of -inf weigh 0 as soon as the row has a
+finite one, in whichever batch that comes.
 """
 import numpy as np
 import pytest
@@ -11,6 +12,7 @@ import torch
 
 import gatgpu
 from gatgpu import inputs
+from test_gpu_row_groups import check_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -102,3 +104,43 @@ def test_infinite_feature_reaches_its_neighbours_only(ctx, K, d):
         out = ctx.stage(0, "out")
         assert np.all(out[hit, 0] == np.inf)
         assert np.all(np.isfinite(out[~hit])) and np.all(np.isfinite(out[:, 1:]))
+
+
+@pytest.mark.parametrize("K,d", SHAPES)
+@pytest.mark.parametrize("precision", [gatgpu.FP32, gatgpu.BF16])
+def test_scores_of_minus_infinity(ctx, K, d, precision):
+    """R of some nodes overflows to -inf with Z and L finite; rows begin with 1 to 300 of them.  Rows
+    of nothing else have no softmax: NaN, as exp(-inf - -inf) is."""
+    n, D, low = 600, 24, 100  # nodes [0, low) have R = -inf
+    rng = np.random.default_rng(K * 64 + d)
+    rows = [[i % low if i < 40 else low + i] for i in range(200)]  # light rows of one edge
+    for before in (1, 3, 4, 7, 8, 9, 16, 63, 64, 65, 128, 200, 300):
+        for after in (0, 1, 4, 8, 40, 130):
+            rows.append(np.concatenate([rng.integers(0, low, before), rng.integers(low, n, after)]))
+    rows += [rng.integers(0, n, k) for k in rng.integers(1, 30, n - len(rows))]
+    row, col = graph_of(rows)
+    p = inputs.glorot_param(D, K, d, 6)
+    x = inputs.normal((n, D), 5)
+    for h in range(K):  # one feature of each head is input h alone, and aR there is huge
+        p["w"][h, :] = 0
+        p["w"][:, h * d] = 0
+        p["w"][h, h * d] = 1
+        x[:, h] = 0
+        x[:low, h] = -100
+    p["al"].reshape(K, d)[:, 0] = 0
+    p["ar"].reshape(K, d)[:, 0] = np.float32(3e38)
+    ctx.set_graph(row, col)
+    ctx.set_layer(0, p)
+    ctx.set_input(x)
+    none = np.array([np.all(np.asarray(r) < low) for r in rows])
+    with np.errstate(invalid="ignore"):
+        for options in OPTIONS:
+            for k, v in options.items():
+                ctx.set_option(k, v)
+            for hidden in (False, True):
+                ctx.layer_forward(0, precision, gatgpu.TRANSFORM_FIRST, hidden)
+                got = {k: ctx.stage(0, k) for k in ("left", "right", "max", "den", "out")}
+                assert np.all(got["right"][:low] == -np.inf) and np.all(np.isfinite(got["right"][low:]))
+                assert np.all(np.isfinite(got["left"]))
+                check_rows(ctx, row, col, K, d, got, hidden, precision == gatgpu.BF16, np.flatnonzero(~none))
+                assert np.all(np.isnan(got["out"][none])) and np.all(np.isnan(got["den"][none]))
