@@ -100,7 +100,7 @@ constexpr uint32_t kPlanMin[kPlans] = {1024, 1536, 2048, 0};
 constexpr uint32_t kPlanChunk[kPlans] = {256, 512, 1024, 0};
 constexpr uint64_t kSmallGraphEdges = 16u << 20, kFineGraphEdges = 1u << 20;
 constexpr uint32_t kSmallPlanMin = 512, kSmallPlanChunk = 256, kFinePlanMin = 128, kFinePlanChunk = 128;
-constexpr uint32_t kBlockMinDefault = 512;  // option GATGPU_OPT_BLOCK_ROW_MIN_DEGREE, unless set
+constexpr uint32_t kBlockMinDefault = 512;  // default of option GATGPU_OPT_BLOCK_ROW_MIN_DEGREE
 constexpr uint64_t kMaxChunksPerRow = 96;
 // Floats per split chunk in SplitTable::part: the widest partial row of the
 // transform-first kernels (512 features, 8 denominators, 8 chunk maxima).
@@ -171,7 +171,6 @@ struct gatgpu_ctx {
     gatgpu::LayerState L[3];
     // options (in-degree thresholds)
     uint32_t block_min = gatgpu::kBlockMinDefault;  // rows below this are never split
-    bool block_min_set = false;      // by the user
     bool fine_split = false;         // kPlanVec and kPlanOne split by kFinePlanMin, kPlanCoarse is built
     uint32_t split_min = 0;          // user option: rows >= this are split (0: per-kernel defaults)
     uint32_t split_chunk = 0;        // user option: edges per chunk (0: per-kernel defaults)

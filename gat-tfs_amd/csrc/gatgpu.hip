@@ -74,7 +74,7 @@ int compute_bins(gatgpu_ctx* c) {
     uint32_t maxdeg = 0;  // degrees are sorted ascending
     if (c->n) HIPCHECK(c, hipMemcpy(&maxdeg, c->sorted_deg + (c->n - 1), 4, hipMemcpyDeviceToHost));
     const bool small = c->e < kSmallGraphEdges;
-    c->fine_split = c->e < kFineGraphEdges && !c->block_min_set && !c->split_min && !c->split_chunk;
+    c->fine_split = c->e < kFineGraphEdges && c->block_min == kBlockMinDefault && !c->split_min && !c->split_chunk;
     const auto fine = [&](int q) { return c->fine_split && (q == kPlanVec || q == kPlanOne); };
     for (int q = 0; q < kPlans; ++q) {
         SplitPlan& P = c->plans[q];
@@ -1245,10 +1245,7 @@ int gatgpu_set_option(gatgpu_ctx* c, int key, int64_t value) {
     if (int r = check_ctx(c)) return r;
     if (value < 0 || value > int64_t(UINT32_MAX)) return fail(c, GATGPU_EINVAL, "option value out of range");
     switch (key) {
-        case GATGPU_OPT_BLOCK_ROW_MIN_DEGREE:
-            c->block_min = uint32_t(value);
-            c->block_min_set = true;
-            break;
+        case GATGPU_OPT_BLOCK_ROW_MIN_DEGREE: c->block_min = uint32_t(value); break;
         case GATGPU_OPT_SPLIT_ROW_MIN_DEGREE:  // 0: the per-kernel defaults
             c->split_min = uint32_t(value);
             break;

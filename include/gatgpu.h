@@ -118,8 +118,8 @@ enum {
     GATGPU_OPT_BLOCK_ROW_MIN_DEGREE = 1, /* rows below are never split (default
                                             512, or 128 on graphs below 1M
                                             edges as long as options 1 to 3
-                                            are at their defaults; 0: no such
-                                            limit)                           */
+                                            are at their defaults, 512 here;
+                                            0: no such limit)                */
     GATGPU_OPT_SPLIT_ROW_MIN_DEGREE = 2, /* rows at/above are split over waves
                                             (default per kernel: 1024 sum form,
                                             1536 8-head, 2048 one-head; 512 on

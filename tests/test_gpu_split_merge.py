@@ -103,3 +103,21 @@ def test_static_layer_takes_the_coarse_split_at_the_limit(ctx):
     small = 20_000  # a graph whose fine split fits reports its larger need, still within the array
     ctx.set_graph(row[:small + 1], np.minimum(col[:int(row[small])], small - 1))
     assert ctx.static_scratch_need(0, gatgpu.BF16, True) <= gatgpu.STATIC_SCRATCH_BYTES
+
+
+def test_options_set_and_restored(ctx):
+    """Options 1 to 3 set and set back to their defaults: the split of a context that never set them
+    (a graph below 1M edges cuts its rows of 128 edges on)."""
+    row, col, _ = chunked_graph(900, 128, (1, 2, 3, 5, 17), 3)
+    ctx.set_graph(row, col)
+    ctx.set_layer(0, inputs.glorot_param(40, 8, 32, 6))
+    need = lambda: ctx.static_scratch_need(0, gatgpu.BF16, True)
+    fresh = need()
+    for k, v, default in ((gatgpu.OPT_BLOCK_ROW_MIN_DEGREE, 600, 512), (gatgpu.OPT_SPLIT_ROW_MIN_DEGREE, 700, 0),
+                          (gatgpu.OPT_SPLIT_CHUNK_EDGES, 512, 0)):
+        ctx.set_option(k, v)
+        assert need() < fresh  # fewer chunks
+        ctx.set_option(k, default)
+        assert need() == fresh
+    ctx.set_option(gatgpu.OPT_BLOCK_ROW_MIN_DEGREE, 512)  # its default, before any other value
+    assert need() == fresh
