@@ -683,6 +683,7 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
         fa.in = D;
         fa.xs = D;
         fa.wpk = Ls.wpk32.as<uint4>();
+        fa.wscale = Ls.wscale32;
         fa.w32 = Ls.w32.as<float>();
         fa.al = Ls.al.as<float>();
         fa.ar = Ls.ar.as<float>();
@@ -940,9 +941,10 @@ int gatgpu_set_layer(gatgpu_ctx* c, int layer, int in, int heads, int dim, const
     HIPCHECK(c, hipMemcpyAsync(L.wq32.p, wq.data(), wn * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(c, hipMemcpyAsync(L.al.p, al, W * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(c, hipMemcpyAsync(L.ar.p, ar, W * 4, hipMemcpyHostToDevice, c->stream));
-    if (const size_t split_bytes = projection_split_bytes(w, in, heads, dim)) {
-        HIPCHECK(c, L.wpk32.ensure(split_bytes));
-        HIPCHECK(c, launch_pack_split(L.w32.as<float>(), in, heads, dim, L.wpk32.p, c->stream));
+    L.wscale32 = projection_split_scale(w, in, heads, dim);
+    if (L.wscale32 > 0.0f) {
+        HIPCHECK(c, L.wpk32.ensure(projection_split_bytes(in, heads, dim)));
+        HIPCHECK(c, launch_pack_split(L.w32.as<float>(), in, heads, dim, L.wscale32, L.wpk32.p, c->stream));
     } else {
         L.wpk32.release();
     }

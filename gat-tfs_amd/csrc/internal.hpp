@@ -276,6 +276,7 @@ struct ProjF32Args {
     uint64_t n;
     int in, xs;
     const uint4* wpk;    // launch_pack_split() order
+    float wscale;        // the factor it was given
     const float* w32;    // [in][width]: the products of rows the split cannot carry
     const float* al;     // aL, aR [width]
     const float* ar;
@@ -290,11 +291,13 @@ struct ProjF32Args {
     // set by the launch: the k range and output blocks of one kernel launch
     int k0, kn, nob;
     bool add;
+    float sum_scale;     // factor of the sums: 1 or 2^48
 };
 hipError_t launch_projection_split(ProjF32Args a, hipStream_t s, int cus);
-size_t projection_split_bytes(const float* w, int in, int heads, int dim);
+float projection_split_scale(const float* w, int in, int heads, int dim);
+size_t projection_split_bytes(int in, int heads, int dim);
 // w: device [in][heads * dim]; out: projection_split_bytes.
-hipError_t launch_pack_split(const float* w, int in, int heads, int dim, void* out, hipStream_t s);
+hipError_t launch_pack_split(const float* w, int in, int heads, int dim, float scale, void* out, hipStream_t s);
 
 // aggregate.hip
 // Rows of at most this many edges share the sum form's 16-edge batches (four

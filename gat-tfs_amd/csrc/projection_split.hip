@@ -4,17 +4,23 @@
 // Reference: projection (baseline/src/baseline_standard.cpp:3-6, cblas_sgemm)
 // and lr_from_z (:7-20).
 //
-// Each FP32 operand is the sum of three bf16 parts, x = x1 + x2 + x3 (x1 the
-// rounding of x, x2 of x - x1, x3 of the rest: exact for normal numbers), and
-// the product keeps the six terms down to 2^-18 of it: x3 w1, x2 w2, x1 w3,
+// Each FP32 operand, times a power of two, is the sum of three bf16 parts, x = x1 +
+// x2 + x3 (x1 the rounding of x, x2 of x - x1, x3 of the rest).  That is exact as
+// long as no part is below bf16's normal range: inputs take 2^24, which keeps the
+// parts of every FP32 number above it, subnormals included (x3 loses bits from
+// 2^-103 down without), and weights 2^-24, which the inputs' factor cancels.  A
+// layer with weights below 2^-79 takes 2^24 for them too, and the sums are brought
+// back once a tile is done (projection_split_scale).
+//
+// The product keeps the six terms down to 2^-18 of it: x3 w1, x2 w2, x1 w3,
 // x2 w1, x1 w2, x1 w1, the small ones first, in one FP32 accumulator chain; the
 // dropped x2 w3 + x3 w2 are below 2^-25 of |x w|.  v_mfma_f32_32x32x16_bf16
 // runs 16 times the rate of v_mfma_f32_32x32x2_f32, so six of them cost 0.38 of
 // the FP32 instruction's time.  Error of the whole forward against 64 bits (2.5M
 // edges): 2.2e-7, 2.5e-7 with the FP32 instruction; over other widths 0.8 to 1.0
-// of it.  On 169K rows: 128 -> 8 x 32 in 78 us (141 with the FP32 instruction),
-// 256 -> 8 x 32 in 127 (251), 256 -> 40 in 69 (93); 120K rows of 100 inputs,
-// which had a VALU product: 61 us (297).  What is left above the 50 to 65 us of
+// of it.  On 169K rows: 128 -> 8 x 32 in 75 us (141 with the FP32 instruction),
+// 256 -> 8 x 32 in 125 (251), 256 -> 40 in 67 (93); 120K rows of 100 inputs,
+// which had a VALU product: 55 us (297).  What is left above the 50 to 65 us of
 // memory traffic is the matrix units: 53 us at their peak for 256 inputs.
 //
 // Work split: W-stationary.  A wave keeps one 32-feature output block's three
@@ -33,8 +39,10 @@
 // divide 16: inside the lane.  Other widths: launch_lr_from_z (3 us and a read of
 // Z more).
 //
-// Inputs the split cannot carry (NaN, infinities, magnitudes of 1e38) mark
-// their tile in LDS, and the tile's products are taken again in plain FP32.
+// Values that leave the range (NaN, infinities, inputs of 2^103 and more) leave an
+// infinity or NaN in the accumulators, and so in their dot with aL: the wave that
+// finds one takes its block of the tile again in plain FP32.  (Marks set in LDS
+// while the input was split cost 2 to 4 us of the times above.)
 //
 // More than 256 inputs run as several launches, each adding its k range to the
 // Z the one before left; the last forms L and R.
@@ -50,11 +58,13 @@ typedef float f32x16 __attribute__((__vector_size__(16 * sizeof(float))));
 
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * kWave;
-constexpr float kSplitMax = 1e38f;
+constexpr float kScaleX = 0x1p24f;
 enum { kLrNone = 0, kLrShare = 1, kLrLane = 2 };  // where a launch forms L and R
 
-// x = p[0] + p[1] + p[2], pairs of bf16 (lo = first).
-__device__ inline void split2(float a, float b, uint32_t (&p)[3]) {
+// scale x = p[0] + p[1] + p[2], pairs of bf16 (lo = first).
+__device__ inline void split2(float a, float b, float scale, uint32_t (&p)[3]) {
+    a *= scale;
+    b *= scale;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         p[q] = bf16x2(a, b);
@@ -76,7 +86,6 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     __shared__ float plr[2][kWaves][2][32];       // L and R shares of a wave's rows, two tiles
     __shared__ float alr[2][kWaves][32];          // aL, aR of the group's output blocks
     clear_words(a.clear, a.nclear);
-    __shared__ int bad[3];
     // Beyond 128 inputs the third parts of W (one of the six terms) stay in LDS:
     // 12 KS registers would not leave room for the rest.
     constexpr int WP = KS > 8 ? 2 : 3;
@@ -102,7 +111,6 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
             (&alr[0][0][0])[q] = f < a.width ? (q < 256 ? a.al : a.ar)[f] : 0.0f;
         }
     }
-    if (threadIdx.x < 3) bad[threadIdx.x] = 0;
     __syncthreads();
     // Staging: wave w takes rows 16 (w % 2) .. + 15 of units w / 2 (and w / 2 +
     // 4), four lanes a row (64 bytes); unit u is k step u % CK of tile u / CK.
@@ -127,18 +135,21 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
             to[y] = v;
         }
     };
-    // The loaded values as three parts into a slot; `mark`: their tile's mark.
-    auto stage = [&](const float4 (&from)[UT], int slot, int mark) {
+    // (No constant to the compiler: it would fold the product into both arms of the
+    // load, which then waits: 125 -> 141 us on 169K rows of 256 -> 8 x 32.)
+    float scale_x = kScaleX;
+    asm("" : "+s"(scale_x));
+    // The loaded values as three parts into a slot.
+    auto stage = [&](const float4 (&from)[UT], int slot) {
 #pragma unroll
         for (int y = 0; y < UT; ++y) {
             const float4 v = from[y];
             uint32_t p0[3], p1[3];
-            split2(v.x, v.y, p0);
-            split2(v.z, v.w, p1);
+            split2(v.x, v.y, scale_x, p0);
+            split2(v.z, v.w, scale_x, p1);
 #pragma unroll
             for (int q = 0; q < 3; ++q)
                 xs[slot][w / 2 + 4 * y][q][((sp / 2) * 32 + srow) * 2 + sp % 2] = make_uint2(p0[q], p1[q]);
-            if (!(fabsf(v.x) + fabsf(v.y) + fabsf(v.z) + fabsf(v.w) < kSplitMax)) bad[mark] = 1;
         }
     };
     // L and R of the tile group before: shares summed over a head's blocks.
@@ -156,7 +167,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     // registers) and slot s + 1 + PD requested while slot s multiplies.
     uint64_t tg = blockIdx.x;
     load(tg, 0, pre[0]);
-    stage(pre[0], 0, 0);
+    stage(pre[0], 0);
     if (NCH == 1) load(tg + gridDim.x < groups ? tg + gridDim.x : groups - 1, 0, pre[0]);
 #pragma unroll
     for (int c = 1; c < NCH && c < PD + 1; ++c) load(tg, c, pre[c % PD]);
@@ -176,7 +187,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int f = 32 * ob + 16 * half + r;
-                if (f < a.width) acc[r] = a.z[rs * a.zs + f];
+                if (f < a.width) acc[r] = a.z[rs * a.zs + f] * a.sum_scale;
             }
         }
 #pragma unroll
@@ -186,15 +197,11 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            if (c == 0) {
-                // Every wave has left the tile before: its L and R shares are
-                // whole, and the mark after the next is free.
-                if (threadIdx.x == 0) bad[(it + 2) % 3] = 0;
-                if (LR == kLrShare && prev < groups) store_lr(prev, (it + 1) & 1);
-            }
+            // Every wave has left the tile before: its L and R shares are whole.
+            if (c == 0 && LR == kLrShare && prev < groups) store_lr(prev, (it + 1) & 1);
             {
                 const int cn = (c + 1) % NCH;  // the next slot's part of its tile
-                stage(pre[cn % PD], slot ^ 1, (c + 1 < NCH ? it : it + 1) % 3);
+                stage(pre[cn % PD], slot ^ 1);
                 const int ahead = c + 1 + PD;
                 if (ahead < NCH) load(tg, ahead, pre[cn % PD]);
                 else if (ahead < 2 * NCH) load(nx, ahead - NCH, pre[cn % PD]);
@@ -222,6 +229,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
             }
         }
         if (!act) continue;
+        // NaN or infinite where an accumulator is (a dot of finite values that
+        // overflows by itself only costs the plain products).
+        float over = 0.0f;
         // kLrLane: feature r of the lane ends its head.
         auto lane_lr = [&](int r, float& lv, float& rv) {
             const int f = 32 * ob + 16 * half + r;
@@ -233,31 +243,10 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
             }
             lv = rv = 0.0f;
         };
-        if (bad[it % 3]) {
-            // Plain FP32 products of the tile, one feature at a time.
-            const float* x = a.x + rs * a.xs + a.k0;
-            float lv = 0.0f, rv = 0.0f;
-#pragma unroll 1
-            for (int r = 0; r < 16; ++r) {
-                const int f = 32 * ob + 16 * half + r;
-                if (f >= a.width) break;
-                const float* wk = a.w32 + size_t(a.k0) * a.width + f;
-                float* to = a.z + rs * a.zs + f;
-                float s = a.add ? *to : 0.0f;
-                for (int k = 0; k < a.kn; ++k) s = __builtin_fmaf(x[k], wk[size_t(k) * a.width], s);
-                if (row < a.n) *to = s;
-                if constexpr (LR != kLrNone) {
-                    lv = __builtin_fmaf(s, alr[0][ob - 8 * g][16 * half + r], lv);
-                    rv = __builtin_fmaf(s, alr[1][ob - 8 * g][16 * half + r], rv);
-                }
-                if constexpr (LR == kLrLane) lane_lr(r, lv, rv);
-            }
-            if constexpr (LR == kLrShare) {
-                lv = xor32_add(lv);
-                rv = xor32_add(rv);
-                plr[it & 1][w][half][col] = half ? rv : lv;
-            }
-            continue;
+        if (a.sum_scale != 1.0f) {
+            const float back = 1.0f / a.sum_scale;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[r] *= back;
         }
         if constexpr (LR != kLrNone) {
             float lv = 0.0f, rv = 0.0f;
@@ -268,10 +257,20 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
                 if constexpr (LR == kLrLane) lane_lr(r, lv, rv);
             }
             if constexpr (LR == kLrShare) {
+                over = lv;
                 lv = xor32_add(lv);
                 rv = xor32_add(rv);
                 plr[it & 1][w][half][col] = half ? rv : lv;
             }
+        }
+        if constexpr (LR != kLrShare) {
+            float o2 = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                over = __builtin_fmaf(acc[r], 0.0f, over);
+                o2 = __builtin_fmaf(acc[r + 1], 0.0f, o2);
+            }
+            over += o2;
         }
         // Lane (half, col) holds features 32 ob + 16 half + {0..15} of row
         // col: four 16-byte pieces.  After the transpose lane c of a quad
@@ -301,6 +300,34 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
             if (rj < a.n && f0 < a.width)
                 *reinterpret_cast<uint4*>(a.z + rj * a.zs + f0) = make_uint4(S[j][0], S[j][1], S[j][2], S[j][3]);
         }
+        if (__any(!(fabsf(over) < INFINITY))) {
+            // Plain FP32 products of the block, one feature at a time, from the
+            // first input on (the sums of the launches before are stored over).
+            // Last, so that the chain of `over` holds nothing else up; the
+            // stores above come from other lanes of the wave and go first.
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+            asm volatile("" ::: "memory");
+            const float* x = a.x + rs * a.xs;
+            float lv = 0.0f, rv = 0.0f;
+#pragma unroll 1
+            for (int r = 0; r < 16; ++r) {
+                const int f = 32 * ob + 16 * half + r;
+                if (f >= a.width) break;
+                float s = 0.0f;
+                for (int k = 0; k < a.k0 + a.kn; ++k) s = __builtin_fmaf(x[k], a.w32[size_t(k) * a.width + f], s);
+                if (row < a.n) a.z[row * a.zs + f] = s;
+                if constexpr (LR != kLrNone) {
+                    lv = __builtin_fmaf(s, alr[0][ob - 8 * g][16 * half + r], lv);
+                    rv = __builtin_fmaf(s, alr[1][ob - 8 * g][16 * half + r], rv);
+                }
+                if constexpr (LR == kLrLane) lane_lr(r, lv, rv);
+            }
+            if constexpr (LR == kLrShare) {
+                lv = xor32_add(lv);
+                rv = xor32_add(rv);
+                plr[it & 1][w][half][col] = half ? rv : lv;
+            }
+        }
     }
     if (LR == kLrShare && prev < groups) {
         __syncthreads();
@@ -314,7 +341,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 // consecutive features; zeros past the inputs and the width.  One wave per
 // (launch, block, k step).
 __global__ void __launch_bounds__(kWave) k_pack_split(const float* __restrict__ w, int in, int width, int ks,
-                                                      uint4* __restrict__ out) {
+                                                      float scale, uint4* __restrict__ out) {
     const int l = threadIdx.x, c = l % 32, hb = (width + 31) / 32;
     const int step = blockIdx.x % ks, b = blockIdx.x / ks % hb, pass = blockIdx.x / ks / hb;
     const int f = 32 * b + 16 * ((c % 8) / 4) + 4 * (c / 8) + c % 4;
@@ -324,7 +351,7 @@ __global__ void __launch_bounds__(kWave) k_pack_split(const float* __restrict__ 
         const int k = 16 * (pass * ks + step) + 8 * (l / 32) + 2 * x;
         uint32_t p[3];
         split2(k < in && f < width ? w[size_t(k) * width + f] : 0.0f,
-               k + 1 < in && f < width ? w[size_t(k + 1) * width + f] : 0.0f, p);
+               k + 1 < in && f < width ? w[size_t(k + 1) * width + f] : 0.0f, scale, p);
 #pragma unroll
         for (int q = 0; q < 3; ++q) part[q][x] = p[q];
     }
@@ -381,30 +408,40 @@ hipError_t launch_lr(const ProjF32Args& a, int lr, hipStream_t s, int cus) {
 
 }  // namespace
 
-// Bytes of the split weights; 0 when a weight is too large for its first part
-// (the VALU projection takes the layer).  w is the host copy.
-size_t projection_split_bytes(const float* w, int in, int heads, int dim) {
+// The weights' factor (see the top), or 0 when no factor holds them all: then the
+// VALU projection takes the layer.  w is the host copy.
+float projection_split_scale(const float* w, int in, int heads, int dim) {
     const size_t count = size_t(in) * heads * dim;
-    bool fits = true;
-    for (size_t q = 0; q < count; ++q) fits &= std::fabs(w[q]) < kSplitMax;
-    int ks, passes;
-    split_passes(in, ks, passes);
-    return fits ? size_t(passes) * ((heads * dim + 31) / 32) * ks * 3 * kWave * 16 : 0;
+    float most = 0.0f, least = 1.0f;
+    for (size_t q = 0; q < count; ++q) {
+        const float m = std::fabs(w[q]);
+        most = m > most ? m : most;
+        least = m > 0.0f && m < least ? m : least;
+    }
+    if (least >= 0x1p-79f) return 0x1p-24f;      // their last bits stay at 2^-126 or above
+    return most < 0x1p103f ? 0x1p24f : 0.0f;
 }
 
-hipError_t launch_pack_split(const float* w, int in, int heads, int dim, void* out, hipStream_t s) {
+size_t projection_split_bytes(int in, int heads, int dim) {
+    int ks, passes;
+    split_passes(in, ks, passes);
+    return size_t(passes) * ((heads * dim + 31) / 32) * ks * 3 * kWave * 16;
+}
+
+hipError_t launch_pack_split(const float* w, int in, int heads, int dim, float scale, void* out, hipStream_t s) {
     int ks, passes;
     split_passes(in, ks, passes);
     const int frags = passes * ((heads * dim + 31) / 32) * ks;
-    k_pack_split<<<dim3(uint32_t(frags)), kWave, 0, s>>>(w, in, heads * dim, ks, static_cast<uint4*>(out));
+    k_pack_split<<<dim3(uint32_t(frags)), kWave, 0, s>>>(w, in, heads * dim, ks, scale, static_cast<uint4*>(out));
     return hipGetLastError();
 }
 
 hipError_t launch_projection_split(ProjF32Args a, hipStream_t s, int cus) {
     if (a.n == 0) return hipSuccess;
     if (a.in < 1 || a.heads < 1 || a.heads > 8 || a.dim < 1 || a.dim > 64 || a.width != a.heads * a.dim || a.zs % 4 ||
-        a.zs < (a.width + 3) / 4 * 4 || a.tiles != (a.n + 31) / 32 || !a.wpk)
+        a.zs < (a.width + 3) / 4 * 4 || a.tiles != (a.n + 31) / 32 || !a.wpk || !(a.wscale > 0.0f))
         return hipErrorInvalidValue;
+    a.sum_scale = a.wscale * kScaleX;
     int ks, passes;
     split_passes(a.in, ks, passes);
     const uint4* wpk = a.wpk;
