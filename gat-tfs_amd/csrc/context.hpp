@@ -42,7 +42,7 @@ struct LayerState {
     bool set = false;
     int in = 0, heads = 0, dim = 0;
     DevBuf w32, wq32, al, ar;
-    DevBuf wpk32;           // three bf16 parts of W for the FP32 projection; empty: no factor holds the weights
+    DevBuf wpk32;           // three bf16 parts of W for the FP32 projection
     float wscale32 = 0.0f;  // their factor
     DevBuf z32, zbf, left, right, mx, den, out32, outbf, in32, inbf;
     // What the last forward of this layer produced.

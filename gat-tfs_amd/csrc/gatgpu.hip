@@ -649,7 +649,7 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
     if (b.clear && tile) {
         pa.clear = b.counter;
         pa.nclear = b.clear;
-    } else if (b.clear && !(!bf16 && Ls.wpk32.p)) {
+    } else if (b.clear && bf16) {
         HIPCHECK(c, launch_clear_u32(b.counter, b.clear, c->stream));
     }
     if (b.projected) {
@@ -676,7 +676,7 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
             pa.x = srcbf;
         }
         HIPCHECK(c, launch_projection_mfma(pa, c->stream, c->cus));
-    } else if (Ls.wpk32.p) {
+    } else {
         ProjF32Args fa{};
         fa.x = src32;
         fa.n = n;
@@ -700,10 +700,6 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
             fa.nclear = b.clear;
         }
         HIPCHECK(c, launch_projection_split(fa, c->stream, c->cus));
-    } else {
-        HIPCHECK(c, launch_projection(src32, nullptr, Ls.w32.as<float>(), n, D, K, dim, Ls.al.as<float>(),
-                                      Ls.ar.as<float>(), static_cast<float*>(b.z), nullptr, b.left, b.right,
-                                      nullptr, zs, c->stream));
     }
     if (ev_base >= 0) HIPCHECK(c, hipEventRecord(c->ev[ev_base + 2], c->stream));
     // ---- fused prescan + softmax + aggregation + normalise + ELU
@@ -942,12 +938,8 @@ int gatgpu_set_layer(gatgpu_ctx* c, int layer, int in, int heads, int dim, const
     HIPCHECK(c, hipMemcpyAsync(L.al.p, al, W * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHECK(c, hipMemcpyAsync(L.ar.p, ar, W * 4, hipMemcpyHostToDevice, c->stream));
     L.wscale32 = projection_split_scale(w, in, heads, dim);
-    if (L.wscale32 > 0.0f) {
-        HIPCHECK(c, L.wpk32.ensure(projection_split_bytes(in, heads, dim)));
-        HIPCHECK(c, launch_pack_split(L.w32.as<float>(), in, heads, dim, L.wscale32, L.wpk32.p, c->stream));
-    } else {
-        L.wpk32.release();
-    }
+    HIPCHECK(c, L.wpk32.ensure(projection_split_bytes(in, heads, dim)));
+    HIPCHECK(c, launch_pack_split(L.w32.as<float>(), in, heads, dim, L.wscale32, L.wpk32.p, c->stream));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     L.set = true;
     L.prepare_ms = ms_wall(t0, Clock::now());

@@ -209,13 +209,6 @@ hipError_t launch_count_le(const uint32_t* sorted_deg, uint64_t n, const uint32_
 hipError_t launch_widen_bf16(const uint16_t* x, float* y, uint64_t count, hipStream_t s);
 // x [n][d] FP32 -> y [n][dp] bf16 with zero columns d..dp-1 (dp a multiple of 4).
 hipError_t launch_to_bf16_pad(const float* x, uint16_t* y, uint64_t n, int d, int dp, hipStream_t s);
-// Z = X W with the L/R attention dots and the store of Z (FP32 or bf16).
-// X is FP32 (x32 != null) or bf16 bits (xbf != null); W is FP32 values (for
-// the bf16 path: bf16-rounded values).
-hipError_t launch_projection(const float* x32, const uint16_t* xbf, const float* w, uint64_t n,
-                             int in, int heads, int dim, const float* al, const float* ar,
-                             float* z32, uint16_t* zbf, float* left, float* right, float* zscratch,
-                             int zs, hipStream_t s);
 // L and R as dots of the FP32 Z rows (lr_from_z).
 hipError_t launch_lr_from_z(const float* z, uint64_t n, int heads, int dim, int zs, const float* al, const float* ar,
                             float* left, float* right, hipStream_t s);

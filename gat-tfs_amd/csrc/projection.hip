@@ -1,10 +1,9 @@
-// Dense per-layer projection Z = X W_all with the attention dots
-// L[i,h] = Z[i,h,:] . aL[h], R[i,h] = Z[i,h,:] . aR[h].
+// The passes beside the projections: the FP32 -> bf16 convert and its inverse, and
+// the attention dots L[i,h] = Z[i,h,:] . aL[h], R[i,h] = Z[i,h,:] . aR[h] of the
+// FP32 layers whose projection does not form them.
 //
-// Reference: projection (baseline/src/baseline_standard.cpp:3-6, one all-head
-// GEMM, cblas_sgemm or cblas_gemm_bf16bf16f32), lr_from_z (:7-20) and the
-// FP32 -> bf16 RNE convert (baseline/src/common.cpp:80-93).  Takes the FP32
-// layers whose weights projection_split.hip cannot carry.
+// Reference: the FP32 -> bf16 RNE convert (baseline/src/common.cpp:80-93) and
+// lr_from_z (baseline/src/baseline_standard.cpp:7-20).
 #include "internal.hpp"
 
 namespace gatgpu {
@@ -42,61 +41,6 @@ k_widen_bf16(const uint16_t* __restrict__ x, float* __restrict__ y, uint64_t cou
     for (uint64_t i = blockIdx.x * uint64_t(kThreads) + threadIdx.x; i < count;
          i += uint64_t(gridDim.x) * kThreads)
         y[i] = bf16_widen(x[i]);
-}
-
-__device__ inline float ldx(const float* x32, const uint16_t* xbf, uint64_t idx) {
-    return xbf ? bf16_widen(xbf[idx]) : x32[idx];
-}
-
-// 64x64 output tile per block, 16-deep K steps through LDS, 4x4 per thread.
-// X rows index blockIdx.x (2^31 limit), output column tiles blockIdx.y.
-__global__ void __launch_bounds__(kThreads)
-k_gemm_tiled(const float* __restrict__ x32, const uint16_t* __restrict__ xbf, const float* __restrict__ w,
-             float* __restrict__ z, uint64_t n, int D, int W, int zs) {
-    __shared__ float As[16][64 + 4];
-    __shared__ float Bs[16][64];
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    const uint64_t row0 = uint64_t(blockIdx.x) * 64;
-    const int col0 = blockIdx.y * 64;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < D; k0 += 16) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int q = threadIdx.x + kThreads * u;
-            const int r = q / 16, kk = q % 16;
-            const uint64_t gr = row0 + r;
-            const int gk = k0 + kk;
-            As[kk][r] = (gr < n && gk < D) ? ldx(x32, xbf, gr * D + gk) : 0.0f;
-            const int kk2 = q / 64, c = q % 64;
-            const int gk2 = k0 + kk2, gc = col0 + c;
-            Bs[kk2][c] = (gk2 < D && gc < W) ? w[size_t(gk2) * W + gc] : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            float av[4], bv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                av[i] = As[kk][ty * 4 + i];
-                bv[i] = Bs[kk][tx * 4 + i];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] += av[i] * bv[j];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint64_t gr = row0 + ty * 4 + i;
-        if (gr >= n) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int gc = col0 + tx * 4 + j;
-            if (gc < W) z[gr * zs + gc] = acc[i][j];
-        }
-    }
 }
 
 // G lanes per (row, head): the dots of lr_from_z over the FP32 Z row, VEC
@@ -174,22 +118,6 @@ hipError_t launch_lr_from_z(const float* z, uint64_t n, int heads, int dim, int 
                         : lr_from_z_lanes<4, 8>(z, n, heads, dim, zs, al, ar, left, right, s);
     return dim <= 8 ? lr_from_z_lanes<1, 2>(z, n, heads, dim, zs, al, ar, left, right, s)
                     : lr_from_z_lanes<1, 8>(z, n, heads, dim, zs, al, ar, left, right, s);
-}
-
-hipError_t launch_projection(const float* x32, const uint16_t* xbf, const float* w, uint64_t n,
-                             int in, int heads, int dim, const float* al, const float* ar,
-                             float* z32, uint16_t* zbf, float* left, float* right, float* zscratch,
-                             int zs, hipStream_t s) {
-    const int W = heads * dim;
-    float* zf = z32 ? z32 : zscratch;
-    if (!zf) return hipErrorInvalidValue;
-    dim3 grid(uint32_t((n + 63) / 64), uint32_t((W + 63) / 64));
-    k_gemm_tiled<<<grid, kThreads, 0, s>>>(x32, xbf, w, zf, n, in, W, zs);
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    if ((err = launch_lr_from_z(zf, n, heads, dim, zs, al, ar, left, right, s)) != hipSuccess) return err;
-    if (zbf) return launch_to_bf16_pad(zf, zbf, n, zs, zs, s);
-    return hipSuccess;
 }
 
 }  // namespace gatgpu

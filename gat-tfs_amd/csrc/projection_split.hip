@@ -39,10 +39,11 @@
 // divide 16: inside the lane.  Other widths: launch_lr_from_z (3 us and a read of
 // Z more).
 //
-// Values that leave the range (NaN, infinities, inputs of 2^103 and more) leave an
-// infinity or NaN in the accumulators, and so in their dot with aL: the wave that
-// finds one takes its block of the tile again in plain FP32.  (Marks set in LDS
-// while the input was split cost 2 to 4 us of the times above.)
+// Values that leave the range (NaN, infinities, inputs of 2^103 and more, weights
+// of 2^103 beside some below 2^-79) leave an infinity or NaN in the accumulators,
+// and so in their dot with aL: the wave that finds one takes its block of the tile
+// again in plain FP32.  (Marks set in LDS while the input was split cost 2 to 4 us
+// of the times above.)
 //
 // More than 256 inputs run as several launches, each adding its k range to the
 // Z the one before left; the last forms L and R.
@@ -408,18 +409,12 @@ hipError_t launch_lr(const ProjF32Args& a, int lr, hipStream_t s, int cus) {
 
 }  // namespace
 
-// The weights' factor (see the top), or 0 when no factor holds them all: then the
-// VALU projection takes the layer.  w is the host copy.
+// The weights' factor (see the top).  w is the host copy.
 float projection_split_scale(const float* w, int in, int heads, int dim) {
     const size_t count = size_t(in) * heads * dim;
-    float most = 0.0f, least = 1.0f;
-    for (size_t q = 0; q < count; ++q) {
-        const float m = std::fabs(w[q]);
-        most = m > most ? m : most;
-        least = m > 0.0f && m < least ? m : least;
-    }
-    if (least >= 0x1p-79f) return 0x1p-24f;      // their last bits stay at 2^-126 or above
-    return most < 0x1p103f ? 0x1p24f : 0.0f;
+    bool small = false;  // a weight whose last bits would fall below 2^-126
+    for (size_t q = 0; q < count; ++q) small |= w[q] != 0.0f && std::fabs(w[q]) < 0x1p-79f;
+    return small ? 0x1p24f : 0x1p-24f;
 }
 
 size_t projection_split_bytes(int in, int heads, int dim) {

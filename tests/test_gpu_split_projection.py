@@ -66,7 +66,7 @@ def test_magnitudes_beyond_the_split(gpu_ctx, D, K, d):
 
 
 def test_weights_beyond_the_split(gpu_ctx):
-    """A weight no bf16 holds: the layer keeps the VALU projection."""
+    """A weight no bf16 holds."""
     x = inputs.normal((65, 24), 4) * np.float32(1e-3)
     p = inputs.glorot_param(24, 2, 32, 5)
     p["w"][5, 7] = np.float32(3.4e38)
