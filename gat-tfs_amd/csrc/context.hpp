@@ -125,7 +125,6 @@ struct TfBufs {
     float* out32 = nullptr;          // [n][W] + kF32Pad, or null
     uint16_t* outbf = nullptr;       // [n][W] (hidden bf16 layers), or null
     // Split-row scratch; null: the plan's own buffers.
-    float* mchunk = nullptr;
     float* part = nullptr;
     uint32_t* counter = nullptr;
     bool fused_convert_ok = false;   // the FP32 input carries kF32Pad floats past its last row

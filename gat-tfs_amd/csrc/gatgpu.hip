@@ -735,7 +735,6 @@ int run_tf(gatgpu_ctx* c, int l, int precision, bool hidden, const float* src32,
     // kernels the 8-head one.
     const SplitPlan& P = c->plans[b.coarse ? kPlanCoarse : grouped ? kPlanOne : kPlanVec];
     SplitTable t = P.table;
-    if (b.mchunk) t.mchunk = b.mchunk;
     if (b.part) t.part = b.part;
     if (b.counter) t.counter = b.counter;
     if (b.next) {

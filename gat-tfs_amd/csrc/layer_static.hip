@@ -26,7 +26,7 @@ void* g_scratch_ptr[kMaxDevices] = {};
 
 // Byte offsets of the intermediates inside the array (256-byte aligned).
 struct StaticPlan {
-    uint64_t xbf = 0, z = 0, left = 0, right = 0, mx = 0, den = 0, out = 0, mchunk = 0, part = 0, counter = 0;
+    uint64_t xbf = 0, z = 0, left = 0, right = 0, mx = 0, den = 0, out = 0, part = 0, counter = 0;
     uint64_t chunks = 0, bytes = 0;
     bool outbf = false, coarse = false;
 };
@@ -52,12 +52,13 @@ StaticPlan plan_with(const gatgpu_ctx* c, int layer, int precision, bool hidden,
     p.mx = take(at, n * K * 4);
     p.den = take(at, n * K * 4);
     p.outbf = bf16 && hidden;
+    // (Used for an unaligned output only, but always kept: whether a layer fits, and
+    // which split it takes, does not hang on the caller's pointer.)
     p.out = take(at, p.outbf ? n * W * 2 : (n * W + kF32Pad) * 4);
     // Split rows of the 8-head and the one-head kernels' plans (whichever runs).
     p.coarse = coarse;
     p.chunks = coarse ? c->plans[kPlanCoarse].table.chunks
                       : std::max(c->plans[kPlanVec].table.chunks, c->plans[kPlanOne].table.chunks);
-    p.mchunk = take(at, p.chunks * 8 * 4);
     p.part = take(at, p.chunks * kTfPartFloats * 4);
     p.counter = take(at, p.chunks * 4);
     p.bytes = at;
@@ -141,7 +142,6 @@ int gatgpu_layer_forward_static(gatgpu_ctx* c, int layer, int precision, int hid
     b.round_bf16 = direct && p.outbf;
     b.no_xbf = true;
     b.coarse = p.coarse;
-    b.mchunk = reinterpret_cast<float*>(base + p.mchunk);
     b.part = reinterpret_cast<float*>(base + p.part);
     b.counter = reinterpret_cast<uint32_t*>(base + p.counter);
     b.fused_convert_ok = false;  // the caller's rows carry no padding: convert kernel first

@@ -275,10 +275,11 @@ int gatgpu_get_static_times(gatgpu_ctx* ctx, gatgpu_static_times* out);
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops): the
  * transform-first gatgpu_layer_forward of `layer` on device-resident rows,
- * with every intermediate (bf16 input rows, Z, L, R, max, den, the output
- * before its final copy, split-row partial sums and arrival counters) in one
- * static device array of GATGPU_STATIC_SCRATCH_BYTES per GPU, held until the
- * process ends.  It calls no allocator.
+ * with every intermediate (bf16 input rows, Z, L, R, max, den, split-row
+ * partial sums and arrival counters, and room for the output, which is taken
+ * where `out` is not 16-byte aligned and copied from there) in one static
+ * device array of GATGPU_STATIC_SCRATCH_BYTES per GPU, held until the process
+ * ends.  It calls no allocator.
  *   x   device FP32 [n][in], original node order
  *   out device FP32 [n][heads*dim], original node order: the values
  *       gatgpu_get_stage(OUT) returns after gatgpu_layer_forward with the

@@ -121,3 +121,17 @@ def test_options_set_and_restored(ctx):
         assert need() == fresh
     ctx.set_option(gatgpu.OPT_BLOCK_ROW_MIN_DEGREE, 512)  # its default, before any other value
     assert need() == fresh
+
+
+def test_static_need_per_chunk(ctx):
+    """A chunk of a split row takes its partials (528 floats) and an arrival counter, and nothing else."""
+    need = []
+    for counts in ((), (1, 2, 3, 5, 17)):
+        row, col, _ = chunked_graph(900, 128, counts, 3)
+        ctx.set_graph(row, col)
+        ctx.set_layer(0, inputs.glorot_param(40, 8, 32, 6))
+        need.append(ctx.static_scratch_need(0, gatgpu.BF16, True))
+    deg = np.diff(row.astype(np.int64))
+    chunks = int(((deg[deg >= 128] + 127) // 128).sum())
+    up = lambda b: (b + 255) // 256 * 256
+    assert need[1] - need[0] == up(chunks * 528 * 4) + up(chunks * 4)
