@@ -21,10 +21,12 @@ BF16_REL_L2 = 1e-2
 # 0 for the split options restores the per-kernel split plans.
 DEFAULT_OPTIONS = {gatgpu.OPT_BLOCK_ROW_MIN_DEGREE: 512, gatgpu.OPT_SPLIT_ROW_MIN_DEGREE: 0,
                    gatgpu.OPT_SPLIT_CHUNK_EDGES: 0}
-# Schedules that route the small graphs' rows through every kernel variant:
-# default, every row a block (generic path), rows >= 16 split into 64-edge chunks.
+# Schedules that route the small graphs' rows through every kernel variant: the
+# default (128-edge chunks from 128 edges on), the 512/256 split of graphs of 1M
+# edges and more (option 1 off its default), rows >= 16 split into 64-edge chunks.
 SCHEDULES = [{}, {gatgpu.OPT_BLOCK_ROW_MIN_DEGREE: 1},
-             {gatgpu.OPT_SPLIT_ROW_MIN_DEGREE: 16, gatgpu.OPT_SPLIT_CHUNK_EDGES: 64}]
+             {gatgpu.OPT_BLOCK_ROW_MIN_DEGREE: 16, gatgpu.OPT_SPLIT_ROW_MIN_DEGREE: 16,
+              gatgpu.OPT_SPLIT_CHUNK_EDGES: 64}]
 
 
 def run_layer(ctx, row, col, x, p, hidden, precision, options=None, dataflow=gatgpu.TRANSFORM_FIRST):
@@ -95,7 +97,7 @@ def test_degree_schedule_bit_exact(gpu_ctx, case):
 
 # ---------------------------------------------------------------- boundary shapes
 SHAPES = [(D, K, d) for D in (17, 33, 128, 256) for K in (1, 2, 4, 8) for d in (7, 32, 40, 47)]
-# The other input widths of the FP32 MFMA projection (D = 2 KH, KH = 16, 32, 48, 96), up to 8 x 64.
+# Other input widths, up to 8 x 64.
 SHAPES += [(32, 8, 32), (64, 4, 40), (96, 8, 64), (192, 2, 47), (192, 1, 64), (256, 8, 64)]
 
 
@@ -790,15 +792,19 @@ def test_bf16_projection_stages(gpu_ctx, D, K, d):
 # 1021 rows: the last 32-row tile holds 29 rows and its last lane quad one, so
 # the stores that leave whole lines after an in-quad transpose (rows 4a + j
 # written by lane quad a, rows past n repeating row n - 1) meet partial tiles.
+# (Below 65 536 rows one wave an output block takes the layer, from there on one
+# wave a tile with the whole-line stores.)
 ODD_ROWS = inputs.Workload("odd1021", "uniform", 1021, 16, 0, 128, 8, 32, 40)
+ODD_MANY = inputs.Workload("odd66557", "uniform", 66557, 4, 0, 128, 8, 32, 40)
 
 
+@pytest.mark.parametrize("graph", [ODD_ROWS, ODD_MANY], ids=lambda w: w.name)
 @pytest.mark.parametrize("D", [100, 256])
-def test_projection_partial_tiles(gpu_ctx, D):
+def test_projection_partial_tiles(gpu_ctx, graph, D):
     """The 8 x 32 projection (whole-line Z stores, R from the stored Z) on a
     graph whose row count is not a multiple of 32 or 4: the same bounds as on
     whole tiles."""
-    check_bf16_projection(gpu_ctx, ODD_ROWS, D, 8, 32)
+    check_bf16_projection(gpu_ctx, graph, D, 8, 32)
 
 
 # Row counts for the W-stationary 8 x 64 projection: its blocks come in pairs

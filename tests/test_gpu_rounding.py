@@ -6,10 +6,10 @@ bit against rne() on the mantissa-midpoint ties of
 baseline/tests/boundaries.cpp:25-26.  Here every place the path rounds is
 compared bit for bit with the oracle's rne_bits:
 
-* the input conversion (stage XBF): the convert kernels (k_to_bf16,
-  k_to_bf16_pad), the fused conversion inside the fast and the wide bf16
-  projections, and the aggregate-first gather table, on 2^20 random finite
-  bit patterns plus the boundary ties, their tails and the extremes;
+* the input conversion (stage XBF): the convert kernel (k_to_bf16_pad), the
+  fused conversion inside the tile, the fast and the wide bf16 projections,
+  and the aggregate-first gather table, on 2^20 random finite bit patterns and
+  more plus the boundary ties, their tails and the extremes;
 * the Z store of the bf16 projections: rows with one nonzero input, so that
   every Z entry is one exact FP32 product x * w whose rounding is known;
 * the hidden-layer output stores of each aggregation kernel: scores all zero
@@ -67,23 +67,31 @@ def assert_bits_equal(got_bits, want_bits, what):
                     f"got 0x{int(got_bits[tuple(i)]):04x} want 0x{int(want_bits[tuple(i)]):04x}")
 
 
-# (D, K, d, dataflow, keep) -> the rounding site the layer's FP32 input goes through
+MANY = 66_557  # rows from which k_proj_tile leaves a layer to the other projections (8 tiles a CU), and some
+
+# (D, K, d, dataflow, keep, n) -> the rounding site the layer's FP32 input goes through
+# (n None: 2^20 values)
 CONVERT_SITES = [
-    (33, 8, 32, gatgpu.TRANSFORM_FIRST, False),   # k_to_bf16_pad (rows not 16-byte multiples)
-    (256, 8, 32, gatgpu.TRANSFORM_FIRST, False),  # k_to_bf16 (16 k steps x 8 head blocks: not fused)
-    (128, 8, 32, gatgpu.TRANSFORM_FIRST, True),   # fused in k_proj_fast (8 x 32, R from Z)
-    (100, 8, 32, gatgpu.TRANSFORM_FIRST, True),   # fused in k_proj_fast, 7 k steps, tail zeroed
-    (128, 1, 47, gatgpu.TRANSFORM_FIRST, True),   # fused in k_proj_fast, 2 head blocks
-    (128, 8, 64, gatgpu.TRANSFORM_FIRST, True),   # fused in k_proj_wide (two output groups)
-    (100, 8, 32, gatgpu.AGGREGATE_FIRST, False),  # L/R front end writing the gather table (R tail)
-    (128, 8, 64, gatgpu.AGGREGATE_FIRST, False),  # gather table without R tail
-    (64, 4, 32, gatgpu.AGGREGATE_FIRST, False),   # neighbour-step form: k_to_bf16_pad into its rows
+    (33, 8, 32, gatgpu.TRANSFORM_FIRST, False, None),   # k_proj_tile (rows not 16-byte multiples)
+    (256, 8, 32, gatgpu.TRANSFORM_FIRST, False, None),  # k_proj_tile, 16 k steps
+    (128, 8, 32, gatgpu.TRANSFORM_FIRST, True, None),   # k_proj_tile (8 x 32, R from Z)
+    (128, 1, 47, gatgpu.TRANSFORM_FIRST, True, None),   # k_proj_tile, 2 output blocks
+    (200, 4, 32, gatgpu.TRANSFORM_FIRST, False, MANY),  # k_proj_tile (a shape without a path of its own)
+    (33, 8, 32, gatgpu.TRANSFORM_FIRST, False, MANY),   # k_to_bf16_pad (rows not 16-byte multiples)
+    (256, 8, 32, gatgpu.TRANSFORM_FIRST, False, MANY),  # k_to_bf16_pad (16 k steps x 8 head blocks: not fused)
+    (128, 8, 32, gatgpu.TRANSFORM_FIRST, True, MANY),   # fused in k_proj_fast (8 x 32, R from Z)
+    (100, 8, 32, gatgpu.TRANSFORM_FIRST, True, MANY),   # fused in k_proj_fast, 7 k steps, tail zeroed
+    (128, 1, 47, gatgpu.TRANSFORM_FIRST, True, MANY),   # fused in k_proj_fast, 2 head blocks
+    (128, 8, 64, gatgpu.TRANSFORM_FIRST, True, None),   # fused in k_proj_wide (two output groups)
+    (100, 8, 32, gatgpu.AGGREGATE_FIRST, False, None),  # L/R front end writing the gather table (R tail)
+    (128, 8, 64, gatgpu.AGGREGATE_FIRST, False, None),  # gather table without R tail
+    (64, 4, 32, gatgpu.AGGREGATE_FIRST, False, None),   # neighbour-step form: k_to_bf16_pad into its rows
 ]
 
 
-@pytest.mark.parametrize("D,K,d,flow,keep", CONVERT_SITES)
-def test_input_conversion_bit_exact(gpu_ctx, D, K, d, flow, keep):
-    n = (1 << 20) // D + 1
+@pytest.mark.parametrize("D,K,d,flow,keep,n", CONVERT_SITES)
+def test_input_conversion_bit_exact(gpu_ctx, D, K, d, flow, keep, n):
+    n = n or (1 << 20) // D + 1
     x = finite_patterns(n * D, 1000 + D).reshape(n, D)
     row, col = inputs.uniform_graph(n, 4, 7)
     p = inputs.glorot_param(D, K, d, 3)
@@ -100,10 +108,11 @@ def test_input_conversion_bit_exact(gpu_ctx, D, K, d, flow, keep):
     assert_bits_equal(bits(xbf), rne(x), f"convert D={D} {K}x{d} flow={flow}")
 
 
-def test_fused_convert_not_kept_by_default(gpu_ctx):
+@pytest.mark.parametrize("n", [4096, MANY])
+def test_fused_convert_not_kept_by_default(gpu_ctx, n):
     """Without the option the fused projection keeps the rounded rows in
     registers only: no XBF stage, and the same Z bits as with it."""
-    n, D = 4096, 128
+    D = 128
     row, col = inputs.uniform_graph(n, 8, 2)
     x = inputs.normal((n, D), 4)
     p = inputs.glorot_param(D, 8, 32, 5)
@@ -140,18 +149,21 @@ def one_hot_rows(rng, n, D, lo_exp, hi_exp, signed, k0=None):
     return x, k
 
 
-# Shapes by projection kernel: fast (8 x 32 with R from Z; one head with R in
-# the row), wide (8 x 64: two groups; 512 inputs), and the general MFMA kernel.
-Z_SHAPES = [(128, 8, 32), (256, 1, 40), (64, 1, 64), (128, 8, 64), (512, 8, 64), (48, 4, 40), (100, 2, 32)]
+# Shapes by projection kernel: tile, or with many rows fast (8 x 32 with R from
+# Z; one head with R in the row); wide (8 x 64: two groups; 512 inputs) and the
+# general MFMA kernel (8 x 40: two groups).
+Z_SHAPES = [(128, 8, 32, None), (256, 1, 40, None), (64, 1, 64, None), (48, 4, 40, None), (100, 2, 32, None),
+            (128, 8, 32, MANY), (256, 1, 40, MANY), (64, 1, 64, MANY),
+            (128, 8, 64, None), (512, 8, 64, None), (48, 8, 40, None)]
 
 
-@pytest.mark.parametrize("D,K,d", Z_SHAPES)
-def test_projection_z_store_bit_exact(gpu_ctx, D, K, d):
+@pytest.mark.parametrize("D,K,d,n", Z_SHAPES)
+def test_projection_z_store_bit_exact(gpu_ctx, D, K, d, n):
     """Z of a bf16 projection is the RNE of its FP32 accumulator.  With one
     nonzero input per row the accumulator is the exact product x * w
     (8-bit significands, exponents within +-20: no overflow or underflow)."""
     rng = np.random.default_rng(D * 100 + K * 10 + d)
-    n = max(2048, (1 << 19) // (K * d))
+    n = n or max(2048, (1 << 19) // (K * d))
     x, k = one_hot_rows(rng, n, D, -20, 20, True)
     p = inputs.glorot_param(D, K, d, 9)
     p["w"] = bf16_values(rng, (D, K * d), -20, 20, True)
@@ -179,8 +191,10 @@ def zero_attention(p):
     return dict(p, al=np.zeros_like(p["al"]), ar=np.zeros_like(p["ar"]))
 
 
+# 128-edge chunks from 128 edges on, the 512/256 split, rows >= 16 in 64-edge chunks.
 SCHEDULES = [{}, {gatgpu.OPT_BLOCK_ROW_MIN_DEGREE: 1},
-             {gatgpu.OPT_SPLIT_ROW_MIN_DEGREE: 16, gatgpu.OPT_SPLIT_CHUNK_EDGES: 64}]
+             {gatgpu.OPT_BLOCK_ROW_MIN_DEGREE: 16, gatgpu.OPT_SPLIT_ROW_MIN_DEGREE: 16,
+              gatgpu.OPT_SPLIT_CHUNK_EDGES: 64}]
 DEFAULTS = {gatgpu.OPT_BLOCK_ROW_MIN_DEGREE: 512, gatgpu.OPT_SPLIT_ROW_MIN_DEGREE: 0,
             gatgpu.OPT_SPLIT_CHUNK_EDGES: 0}
 
@@ -196,15 +210,14 @@ def run_with(ctx, opts, fn):
 
 
 # Transform-first hidden bf16 layers by aggregation kernel: k_agg_vec (8 x 32
-# with R from Z, 8 x 64), k_agg_k1 (one head, R in the row), the generic
-# wave/block kernels (4 x 40).
+# with R from Z, 8 x 64), k_agg_rows (one head, R in the row; 4 x 40).
 TF_OUT_SHAPES = [(128, 8, 32), (128, 8, 64), (128, 1, 47), (64, 4, 40)]
 
 
 @pytest.mark.parametrize("D,K,d", TF_OUT_SHAPES)
 def test_aggregation_output_store_bit_exact(gpu_ctx, D, K, d):
     """Hidden bf16 outputs are the RNE of the normalised sum: with p = 1 and
-    power-of-two degrees (up to 2048, split and block rows included), the
+    power-of-two degrees (up to 2048, split rows included), the
     value before rounding is sum_j Z_j / deg exactly (Z_j in [1, 4] with
     8-bit significands), whatever the summation order."""
     rng = np.random.default_rng(D + K + d)

@@ -19,13 +19,13 @@ from gatgpu import inputs
 pytestmark = pytest.mark.gpu
 
 # (D, K, d, precision, hidden): the 8-head vector kernel (R from Z; R gathered),
-# the one-head kernel (R in the row), the generic kernels, the FP32 MFMA and
-# tiled projections.
+# the row-group kernel (one head with R in the row; 4 heads), and the FP32
+# projection with L and R formed in it (8 x 32) and after it (2 x 7).
 CASES = [(128, 8, 32, gatgpu.BF16, True), (256, 8, 64, gatgpu.BF16, False), (256, 1, 47, gatgpu.BF16, False),
          (64, 4, 40, gatgpu.BF16, True), (128, 8, 32, gatgpu.FP32, True), (33, 2, 7, gatgpu.FP32, False),
          (256, 1, 47, gatgpu.BF16, True)]
 # Split rows from 16 edges in chunks of 64: the scratch partial sums and counters are used.
-SPLIT = {gatgpu.OPT_SPLIT_ROW_MIN_DEGREE: 16, gatgpu.OPT_SPLIT_CHUNK_EDGES: 64}
+SPLIT = {gatgpu.OPT_BLOCK_ROW_MIN_DEGREE: 16, gatgpu.OPT_SPLIT_ROW_MIN_DEGREE: 16, gatgpu.OPT_SPLIT_CHUNK_EDGES: 64}
 
 
 def graphs():
