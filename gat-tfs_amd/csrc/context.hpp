@@ -78,9 +78,8 @@ struct LayerState {
 // a short launch (169K-node, 2.5M-edge power-law graph: 0.88 ms against 1.23
 // with the plans above).  Graphs with heavier rows scale a plan (chunk and
 // min) by the smallest power of two that keeps the heaviest row within
-// kMaxChunksPerRow chunks: each chunk reduces the maxima of all chunks of its
-// row and the last one adds all partial sums, so many chunks per row cost
-// more than they balance.  The 8-head kernel (one row per wave) scales min
+// kMaxChunksPerRow chunks: the last chunk of a row adds all its partial sums,
+// so many chunks per row cost more than they balance.  The 8-head kernel (one row per wave) scales min
 // with the chunk; the sum form (32-row tiles) holds a heavy row's neighbours
 // at the same pace, and it and the row-group kernel split from twice the chunk
 // instead.  On the 100M-edge R-MAT graph (max in-degree
@@ -162,7 +161,6 @@ struct gatgpu_ctx {
     std::vector<uint32_t> perm_h;
     uint64_t neighbor_steps = 0;
     uint32_t max_degree = 0;
-    gatgpu::RowBins bins;
     // input
     bool input = false;
     int din = 0;

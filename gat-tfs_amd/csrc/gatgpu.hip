@@ -98,15 +98,15 @@ int compute_bins(gatgpu_ctx* c) {
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     RowBins b;
     b.n = c->n;
-    b.block_begin = c->block_min ? pos[0] : 0;
     b.short_end = pos[1 + kPlans];
     b.wave_begin = pos[2 + kPlans];
-    c->bins = b;
+    // Rows below option 1 are not split (the fine split's own floor is lower).
+    const uint64_t block_begin = c->block_min ? pos[0] : 0;
     std::vector<uint64_t> prow;
     for (int q = 0; q < kPlans; ++q) {
         SplitPlan& P = c->plans[q];
         P.bins = b;
-        P.bins.split_begin = pos[1 + q] < b.block_begin && !fine(q) ? b.block_begin : pos[1 + q];
+        P.bins.split_begin = pos[1 + q] < block_begin && !fine(q) ? block_begin : pos[1 + q];
         if (q == kPlanCoarse && !c->fine_split) {  // nobody takes it
             P.table = SplitTable{};
             continue;

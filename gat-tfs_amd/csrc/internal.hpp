@@ -308,9 +308,8 @@ constexpr uint64_t kWaveDegEdges = 1u << 21;  // graphs of fewer edges take kWav
 struct RowBins {
     // Sorted positions split by degree: [0, short_end): rows of at most
     // kShortDeg edges; [wave_begin, n): of kWaveDeg edges or more;
-    // [split_begin, n): cut into chunks (never below block_begin, the first
-    // row of GATGPU_OPT_BLOCK_ROW_MIN_DEGREE edges).
-    uint64_t block_begin = 0, split_begin = 0, n = 0, short_end = 0, wave_begin = 0;
+    // [split_begin, n): cut into chunks.
+    uint64_t split_begin = 0, n = 0, short_end = 0, wave_begin = 0;
 };
 struct AggArgs {
     const uint64_t* prow;
