@@ -33,10 +33,10 @@
 //   * lighter rows: one group each, 64 / G rows of (nearly) equal degree a wave.
 // Measured against one group per row up to the split degree, and one wave (or
 // block) per row with the scores exchanged through LDS for the other widths:
-// 169K nodes / 2.5M edges, one head of 40: bf16 155 -> 71 us, FP32 161 -> 109;
-// 60K / 1.2M, one head of 47: 95 -> 31 us; 20K / 300K, 4 heads of 16, FP32:
-// 247 -> 19 us; 20K / 160K, 8 heads of 8, bf16: 56 -> 9 us; R-MAT 2^20 / 24M,
-// one head of 16: 710 -> 541 us.
+// 169K nodes / 2.5M edges, one head of 40: bf16 155 -> 49 us, FP32 161 -> 87;
+// 60K / 1.2M, one head of 47: 95 -> 27 us; 20K / 300K, 4 heads of 16, FP32:
+// 247 -> 16 us; 20K / 160K, 8 heads of 8, bf16: 56 -> 11 us; R-MAT 2^20 / 24M,
+// one head of 16: 710 -> 355 us.
 #include "internal.hpp"
 
 namespace gatgpu {
