@@ -260,7 +260,7 @@ __device__ inline void edges(const GrpArgs<typename C::ZT>& a, Lane<C>& s, uint6
     const uint32_t lane_t = s.sub < C::B ? uint32_t(s.sub) : 0u;
     auto id_at = [&](uint32_t q) { return ids[q < total ? q : total - 1]; };
     uint32_t next = id_at(start + lane_t);
-    for (uint32_t done = start; done < total; done += step) {
+    for (uint32_t done = start;; done += step) {
         const uint32_t left = total - done;
         const int cnt = left < uint32_t(C::B) ? int(left) : C::B;
         const uint32_t j = next;  // past the end: the last source
@@ -269,6 +269,7 @@ __device__ inline void edges(const GrpArgs<typename C::ZT>& a, Lane<C>& s, uint6
         // of a skewed graph have a few edges only.
         if (left > uint32_t(C::B) / 2) batch<C, C::B, C::B / 2 + 1>(a, s, j, cnt);
         else batch<C, C::B / 2, 1>(a, s, j, cnt);
+        if (left <= step) return;  // (not done + step < total: that sum may pass 2^32)
     }
 }
 
