@@ -44,10 +44,6 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWavesPerBlock = kThreads / kWave;
-// A row's maximum before its first edge: finite, so that scores of -inf weigh
-// exp(-inf - kNoMax) = 0 while nothing else was met (from -inf they would weigh
-// exp(-inf + inf), NaN, and with them the row).
-constexpr float kNoMax = -3.402823466e38f;
 constexpr uint32_t kPartStride = 512 + 16;  // sums, denominators of the heads, maxima of the heads
 
 template <int BYTES>
@@ -299,8 +295,7 @@ __device__ inline void finish(const GrpArgs<typename C::ZT>& a, const Lane<C>& s
     constexpr int V = C::VEC;
 #pragma unroll
     for (int v = 0; v < C::VPL; ++v) {
-        // Nothing but scores of -inf (or NaN): no softmax, as exp(-inf - max) is NaN.
-        const bool none = any && s.m[v] == kNoMax && !(s.d[v] > 0.0f);
+        const bool none = any && no_softmax(s.m[v], s.d[v]);
         const float d = none ? NAN : s.d[v];
         if (s.lead[v]) {
             a.mx[uint64_t(i) * a.K + s.head[v]] = none ? -INFINITY : any ? s.m[v] : 0.0f;

@@ -131,7 +131,7 @@ __device__ inline void batch_sums(const uint4 (&z)[C::U][C::VPL], const float (&
             mb = ok[u] ? mx : mb;
         }
         const float mn = max_quiet(st.m[v], mb);
-        const float sc = mn > st.m[v] ? exp_w(st.m[v] - mn) : 1.0f;  // exp(-inf) = 0 on a slot's first edge
+        const float sc = mn > st.m[v] ? exp_w(st.m[v] - mn) : 1.0f;  // 0 on a slot's first edge (m = kNoMax)
         st.m[v] = mn;
         st.den[v] *= sc;
 #pragma unroll
@@ -175,11 +175,9 @@ __device__ inline void load_ids(const uint32_t* __restrict__ pcol, uint64_t base
 // the slot-0 / slot-1 sources j0, j1 of a load (RB bytes per row; smask all
 // ones in the slot-1 lanes), two VALU operations on scalar operands instead
 // of a per-lane select and a 64-bit address.
-// FREE (RZ): every edge slot has seen a valid edge before its first past-end
-// edge (the row has at least EPI edges, or m starts at a chunk's finite row
-// max), so m is finite there: a past-end edge is given the score -inf, which
-// leaves m in place (scale e^0 = 1) and weighs 0 -- the values of the tested
-// form, without its selects.
+// FREE (RZ, rows of at least EPI edges): a past-end edge is given the score
+// -inf, which leaves m, finite from the start (kNoMax), in place (scale e^0 = 1)
+// and weighs 0 -- the values of the tested form, without its selects.
 template <class C, class ZT, bool RZ, bool O32 = false, bool FREE = false>
 __device__ inline void batch(uint32_t left, const uint32_t (&js)[C::BATCH], const float* __restrict__ R,
                              const ZT* __restrict__ Z, int slot, int sub, Lane<C>& st) {
@@ -249,12 +247,12 @@ __device__ inline void batch(uint32_t left, const uint32_t (&js)[C::BATCH], cons
             if constexpr (FREE) {
                 const float sv = ok[u] ? sc_ : -INFINITY;
                 mn = max_quiet(st.m[0], sv);
-                scale = exp_w(st.m[0] - mn);  // exactly 1 when m stays; 0 on a slot's first edge
+                scale = exp_w(st.m[0] - mn);  // exactly 1 when m stays; 0 on a slot's first edge (m = kNoMax)
                 p = exp_w(sv - mn);           // 0 past the end
             } else {
                 const float mx = max_quiet(st.m[0], sc_);  // unconditional: no branch around the asm
                 mn = ok[u] ? mx : st.m[0];
-                scale = mn > st.m[0] ? exp_w(st.m[0] - mn) : 1.0f;  // exp(-inf) = 0 on a slot's first edge
+                scale = mn > st.m[0] ? exp_w(st.m[0] - mn) : 1.0f;  // 0 on a slot's first edge
                 p = ok[u] ? exp_w(sc_ - mn) : 0.0f;
             }
             if (__any(scale != 1.0f)) {
@@ -352,11 +350,12 @@ __device__ inline void finish_row(uint32_t i, const float (&acc)[C::ACC], const 
 #pragma unroll
     for (int v = 0; v < C::VPL; ++v) {
         const int f0 = (sub + kWave * v) * C::VEC;
+        const bool none = no_softmax(M[v], den[v]);  // (an empty row's M is 0)
         if (f0 % C::DIM == 0) {
-            mx[uint64_t(i) * C::K + h[v]] = M[v];
-            dn[uint64_t(i) * C::K + h[v]] = den[v];
+            mx[uint64_t(i) * C::K + h[v]] = none ? -INFINITY : M[v];
+            dn[uint64_t(i) * C::K + h[v]] = none ? NAN : den[v];
         }
-        const float scale = den[v] > 0.0f ? 1.0f / den[v] : 0.0f;
+        const float scale = none ? NAN : den[v] > 0.0f ? 1.0f / den[v] : 0.0f;
         float o[C::VEC];
 #pragma unroll
         for (int x = 0; x < C::VEC; ++x) o[x] = acc[v * C::VEC + x] * scale;
@@ -469,7 +468,7 @@ __device__ inline void run_chunk(const VArgs<ZT>& a, uint64_t c, int lane, int s
 #pragma unroll
     for (int v = 0; v < C::VPL; ++v) {
         st.L[v] = a.L[uint64_t(i) * C::K + st.h[v]];
-        st.m[v] = -INFINITY;
+        st.m[v] = kNoMax;
     }
     aggregate<C, ZT, RZ, O32>(beg, end, a.pcol, a.R, a.Z, slot, sub, st);
     constexpr int PF = part_floats<C>();
@@ -552,7 +551,7 @@ __global__ void __launch_bounds__(kThreads) k_agg_vec(VArgs<ZT> a, uint64_t shor
 #pragma unroll
     for (int v = 0; v < C::VPL; ++v) {
         st.L[v] = a.L[uint64_t(i) * C::K + st.h[v]];
-        st.m[v] = -INFINITY;
+        st.m[v] = kNoMax;
     }
     aggregate<C, ZT, RZ, O32>(beg, end, a.pcol, a.R, a.Z, slot, sub, st);
     // Empty row: max 0, denominator 0, output 0 (baseline/src/ref_fp32.cpp:11).
@@ -608,7 +607,7 @@ __global__ void __launch_bounds__(kThreads) k_agg_vec_short(VArgs<uint16_t> a, u
     for (int r = 0; r < RW; ++r) {
         init_lane<C, uint16_t, false>(a, sub, st[r]);
         st[r].L[0] = a.L[uint64_t(ri[r] == kNone ? 0u : ri[r]) * C::K + st[r].h[0]];
-        st[r].m[0] = -INFINITY;
+        st[r].m[0] = kNoMax;
         uint32_t js[C::BATCH], jc[C::BATCH];
         load_ids<C>(a.pcol, rb[r], js);
         jc[0] = js[0];
@@ -695,11 +694,12 @@ template <class C>
 __device__ inline void finish_row_tile(const Lane<C>& st, const float (&tot)[4], int slot, int sub,
                                        float* smd, unsigned char* trow) {
     static_assert(C::VEC == 8 && C::VPL == 1 && C::W == 256, "bf16 8 x 32 rows");
+    const bool none = no_softmax(st.m[0], st.den[0]);
     if (slot == 0 && (sub * C::VEC) % C::DIM == 0) {
-        smd[st.h[0]] = st.m[0];
-        smd[kNextTile * C::K + st.h[0]] = st.den[0];
+        smd[st.h[0]] = none ? -INFINITY : st.m[0];
+        smd[kNextTile * C::K + st.h[0]] = none ? NAN : st.den[0];
     }
-    const float scale = st.den[0] > 0.0f ? 1.0f / st.den[0] : 0.0f;
+    const float scale = none ? NAN : st.den[0] > 0.0f ? 1.0f / st.den[0] : 0.0f;
     const uint32_t w0 = bf16x2(elu_bf16(tot[0] * scale), elu_bf16(tot[1] * scale));
     const uint32_t w1 = bf16x2(elu_bf16(tot[2] * scale), elu_bf16(tot[3] * scale));
     *reinterpret_cast<uint2*>(trow + 16 * sub + 8 * slot) = make_uint2(w0, w1);
@@ -737,7 +737,7 @@ k_agg_vec_next(VArgs<uint16_t> a, NextProj f, uint64_t chunk_blocks) {
                 Lane<C> st;
                 init_lane<C, uint16_t, true>(a, sub, st);
                 st.L[0] = a.L[k * C::K + st.h[0]];
-                st.m[0] = -INFINITY;
+                st.m[0] = kNoMax;
                 aggregate<C, uint16_t, true, O32, false, false>(beg, end, a.pcol, a.R, a.Z, slot, sub, st);
                 float tot[4];
                 merge_slots_split<C>(st, tot);

@@ -90,6 +90,13 @@ __device__ inline float elu(float x) { return x >= 0.0f ? x : expm1f(x); }
 // wherever e^x is above 2^-30.
 __device__ inline float exp_w(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
 
+// The online softmax's maximum before a row's (or chunk's) first edge: finite, so
+// that scores of -inf weigh exp(-inf - kNoMax) = 0 while nothing else was met (from
+// -inf they would weigh exp(-inf + inf), NaN, and with them the row).
+constexpr float kNoMax = -3.402823466e38f;
+// A row with nothing but scores of -inf (or NaN): no softmax, NaN as exp(-inf - max) is.
+__device__ inline bool no_softmax(float m, float den) { return m == kNoMax && !(den > 0.0f); }
+
 // ELU for outputs that are stored as bf16: e^x - 1 from the hardware exp2
 // (exp_w) where x < -1/8 (there |e^x - 1| > 0.11, so the exp2 error stays
 // below 2e-6 of the result), and from the Taylor polynomial of e^x - 1 to

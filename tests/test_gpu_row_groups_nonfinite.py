@@ -1,4 +1,5 @@
-"""The row-group aggregation (csrc/aggregate.hip) on values that are not finite.
+"""The transform-first aggregations (csrc/aggregate.hip; -inf scores also csrc/aggregate_vec.hip) on
+values that are not finite.
 
 A batch's lanes past the row's last edge must not carry
 another row's infinity or NaN into a row that is not connected to it; a row
@@ -106,17 +107,21 @@ def test_infinite_feature_reaches_its_neighbours_only(ctx, K, d):
         assert np.all(np.isfinite(out[~hit])) and np.all(np.isfinite(out[:, 1:]))
 
 
-@pytest.mark.parametrize("K,d", SHAPES)
+@pytest.mark.parametrize("K,d", SHAPES + [(8, 32), (8, 64)])
 @pytest.mark.parametrize("precision", [gatgpu.FP32, gatgpu.BF16])
 def test_scores_of_minus_infinity(ctx, K, d, precision):
-    """R of some nodes overflows to -inf with Z and L finite; rows begin with 1 to 300 of them.  Rows
-    of nothing else have no softmax: NaN, as exp(-inf - -inf) is."""
+    """R of some nodes overflows to -inf with Z and L finite; rows begin with 1 to 300 of them, or have
+    them where a chunk of the row begins.  Rows of nothing else have no softmax: NaN, as
+    exp(-inf - -inf) is."""
     n, D, low = 600, 24, 100  # nodes [0, low) have R = -inf
     rng = np.random.default_rng(K * 64 + d)
     rows = [[i % low if i < 40 else low + i] for i in range(200)]  # light rows of one edge
     for before in (1, 3, 4, 7, 8, 9, 16, 63, 64, 65, 128, 200, 300):
         for after in (0, 1, 4, 8, 40, 130):
             rows.append(np.concatenate([rng.integers(0, low, before), rng.integers(low, n, after)]))
+    for lows in (1, 2, 16, 128, 150):
+        for chunk in (64, 128, 256):
+            rows.append(np.concatenate([rng.integers(low, n, chunk), rng.integers(0, low, lows), rng.integers(low, n, 200)]))
     rows += [rng.integers(0, n, k) for k in rng.integers(1, 30, n - len(rows))]
     row, col = graph_of(rows)
     p = inputs.glorot_param(D, K, d, 6)
